@@ -13,13 +13,37 @@ constexpr int kAbsBlocks = WFB_ABSMEAN_WS_DOUBLES;
 
 // Stage 1: block b sums |w| over the grid-stride set {i : i % (blocks*256) in block b's range},
 // in fp64, each thread sequentially, then a fixed tree.  Deterministic for a given numel.
+// Bound by how many loads are in flight (one dependent fp64 add per element hides none): a thread requests
+// kAbsBatch elements before it adds the first, in the same order as one at a time, so the sum keeps its bits.
+// The last elements are taken kAbsTail at a time from clamped indices, those past the end adding +0.0 (which
+// leaves a non-negative sum as it is): a guard around each load would wait for each.
+// 14336 x 4096 fp32: 103 -> 42 us (5.6 TB/s), 6912 x 2560 bf16 21.9 -> 8.6 us (traced).
+constexpr int kAbsBatch = 16, kAbsTail = 4;
+
 template <int DT>
 __global__ __launch_bounds__(256) void absmean_partial_kernel(const void* __restrict__ w, int64_t numel,
                                                               double* __restrict__ partial) {
   __shared__ double red[256];
+  constexpr int64_t kStride = (int64_t)kAbsBlocks * 256;
   double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < numel; i += (int64_t)kAbsBlocks * 256)
-    acc += (double)fabsf(load_elem<DT>(w, i));
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (; i + (kAbsBatch - 1) * kStride < numel; i += kAbsBatch * kStride) {
+    float v[kAbsBatch];
+#pragma unroll
+    for (int u = 0; u < kAbsBatch; ++u) v[u] = load_elem<DT>(w, i + u * kStride);
+#pragma unroll
+    for (int u = 0; u < kAbsBatch; ++u) acc += (double)fabsf(v[u]);
+  }
+  for (; i < numel; i += kAbsTail * kStride) {
+    float v[kAbsTail];
+#pragma unroll
+    for (int u = 0; u < kAbsTail; ++u) {
+      const int64_t j = i + u * kStride;
+      v[u] = load_elem<DT>(w, j < numel ? j : numel - 1);
+    }
+#pragma unroll
+    for (int u = 0; u < kAbsTail; ++u) acc += i + u * kStride < numel ? (double)fabsf(v[u]) : 0.0;
+  }
   red[threadIdx.x] = acc;
   __syncthreads();
   for (int o = 128; o >= 1; o >>= 1) {
