@@ -372,6 +372,21 @@ int wfb_linear_i2s_glu(const uint8_t* qweight, int64_t n, int64_t k, const int8_
                        const float* a_scale, const float* w_scales_dev, int act_kind, int mid_dtype, float* out,
                        int64_t ldo, void* stream);
 
+/* Gradients of the straight-through linear (WF/models/bitlinear.py:86-113) at the quantised operands:
+ *   grad_x[m, k] = w_scale * sum_n g[m, n] * t[n, k]                    (wfb_linear_grad_x, t the ternary weight)
+ *   grad_w[n, k] = sum_m (g[m, n] * a_scale[m]) * act[m, k]             (wfb_linear_grad_w, act the int8 codes)
+ * for k < K (K <= k_pad, the packed row length), in fp32: every product is exact, g * a_scale is rounded once to
+ * fp32 and the sums are fp32.  g: fp32 / bf16 / fp16 [M, N], row stride ldg; w_scale_dev, a_scale: fp32 on the
+ * device; out: fp32 / bf16 / fp16, row stride ldo.  work: 16-byte aligned device memory of at least the bytes
+ * wfb_linear_grad_workspace reports (host only, no GPU work).  M, N, K >= 1 and below 2^20 each. */
+int wfb_linear_grad_workspace(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* bytes_x, int64_t* bytes_w);
+int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const uint8_t* qweight,
+                      int64_t k, int64_t k_pad, const float* w_scale_dev, void* out, int out_dtype, int64_t ldo,
+                      void* work, void* stream);
+int wfb_linear_grad_w(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const int8_t* act, int64_t lda,
+                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* work,
+                      void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,74 @@
+"""Gradient kernels of the straight-through linear (linear_grad_x / linear_grad_w) against float64 products of the
+same codes and scales: edges of the 64 / 128 / 256-row tiles, rows that are not 16-byte aligned, every gradient type,
+sums short enough for one stage and long enough to be split.
+
+Bound: every product is exact in fp32 and the sums are fp32, so the normwise error is that of an fp32 sum of C terms,
+at most about sqrt(3 C / 16) roundings of 2^-24 (three planes, 16 terms per matrix instruction) plus the rounding of
+g * a_scale and the result's own: below 1e-6 for C <= 2048 (measured 0.3-4e-7); 16-bit outputs are the fp32 result
+rounded once, bit for bit."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 128), (5, 257, 129), (63, 65, 512), (129, 1000, 640), (300, 96, 2057),
+                                   (2048, 136, 257), (70, 2040, 384)])
+def test_linear_grads_match_float64(pkg, dev, m, n, k, dtype):
+    ops = pkg.ops
+    g = torch.Generator(device=dev).manual_seed(m * n + k)
+    rand = lambda *s: torch.randn(s, generator=g, device=dev)  # noqa: E731
+    k_pad = (k + 127) // 128 * 128
+    qw, scale = ops.pack_ternary_i2s((rand(n, k) * 0.02), k_pad=k_pad)
+    codes, a_scale = ops.quantize_activations_i8_per_token(rand(m, k) * (1 + rand(m, 1).abs()), k_pad=k_pad)
+    gy = rand(m, n).to(dtype)
+    t = ops.unpack_i2s(qw)[:, :k].double()
+    gx = ops.linear_grad_x(qw, scale, gy, k, torch.float32)
+    gw = ops.linear_grad_w(codes, a_scale, gy, k, torch.float32)
+    assert _rel(gx, (gy.double() @ t) * scale.double()) <= 1e-6
+    assert _rel(gw, (gy.double() * a_scale.double()[:, None]).t().contiguous() @ codes[:, :k].double()) <= 1e-6
+    for out in (torch.bfloat16, torch.float16):
+        assert torch.equal(ops.linear_grad_x(qw, scale, gy, k, out), gx.to(out))
+        assert torch.equal(ops.linear_grad_w(codes, a_scale, gy, k, out), gw.to(out))
+
+
+def test_non_finite_gradients_reach_the_products(pkg, dev):
+    """An infinite or NaN gradient gives what an fp32 product gives: inf * code, NaN where a code is 0."""
+    ops = pkg.ops
+    m, n, k = 6, 40, 256
+    g = torch.Generator(device=dev).manual_seed(3)
+    qw, scale = ops.pack_ternary_i2s(torch.randn((n, k), generator=g, device=dev))
+    codes, a_scale = ops.quantize_activations_i8_per_token(torch.randn((m, k), generator=g, device=dev))
+    gy = torch.randn((m, n), generator=g, device=dev)
+    gy[1, 3], gy[4, 7] = float("inf"), float("nan")
+    gx = ops.linear_grad_x(qw, scale, gy, k, torch.float32)
+    gw = ops.linear_grad_w(codes, a_scale, gy, k, torch.float32)
+    ex = (gy.double() @ ops.unpack_i2s(qw).double()) * scale.double()
+    ew = (gy.double() * a_scale.double()[:, None]).t().contiguous() @ codes.double()
+    for got, want in ((gx, ex), (gw, ew)):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        fine = want.isfinite()
+        assert torch.allclose(got[fine].double(), want[fine], rtol=0, atol=1e-5 * float(want[fine].abs().max()))
+
+
+def test_gradients_of_gradients_and_batched_gradients_keep_working(pkg, dev):
+    """create_graph and is_grads_batched go through the torch products that autograd and vmap see through."""
+    torch.manual_seed(5)
+    mod = pkg.BitLinear(256, 96, device=dev)
+    x = torch.randn(7, 256, device=dev, requires_grad=True)
+    gy = torch.randn(7, 96, device=dev, requires_grad=True)
+    plain = torch.autograd.grad(mod(x), [x, mod.weight], gy.detach())
+    (gx,) = torch.autograd.grad(mod(x), x, gy, create_graph=True)
+    (ggy,) = torch.autograd.grad(gx.square().sum(), gy)
+    w = pkg.unpack_i2s(mod.qweight)[:, :256].float() * mod.weight_scale
+    assert _rel(gx.detach(), plain[0].double()) <= 1e-6
+    assert _rel(ggy, 2 * (gx.detach() @ w.t()).double()) <= 1e-5
+    both = torch.stack([gy.detach(), 2 * gy.detach()])
+    bx, bw = torch.autograd.grad(mod(x), [x, mod.weight], both, is_grads_batched=True)
+    assert _rel(bx[0], plain[0].double()) <= 1e-6 and _rel(bw[1], 2 * plain[1].double()) <= 1e-6

@@ -31,6 +31,9 @@ import torch.nn as nn
 from .ops import (
     QK_I2_S,
     bitnet_linear,
+    linear_grad_supported,
+    linear_grad_w,
+    linear_grad_x,
     pack_ternary_i2s,
     quantize_activations_i8,
     quantize_activations_i8_per_token,
@@ -66,6 +69,13 @@ def _out_dtype(x: torch.Tensor) -> torch.dtype:
     return torch.float32 if x.dtype == torch.float32 else torch.bfloat16
 
 
+def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
+    """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
+    backward is itself being differentiated (create_graph) or batched by a functorch transform: those take the torch
+    products, which autograd and vmap see through."""
+    return not torch.is_grad_enabled() and linear_grad_supported(gy, in_features)
+
+
 class _BitLinearSTE(torch.autograd.Function):
     """Straight-through estimator of the reference training forward at lambda = 1
     (WF/models/bitlinear.py:86-113).  Forward: the kernels' quantised product (per-token int8 codes of x,
@@ -85,8 +95,17 @@ class _BitLinearSTE(torch.autograd.Function):
     def backward(ctx, gy):
         q, a_scale, qweight, wscale = ctx.saved_tensors
         xdt, wdt, bdt, kin = ctx.meta
-        g = gy.to(torch.float32).contiguous()
         gx = gw = gb = None
+        if _kernel_grads(gy, kin):
+            gy = gy.contiguous()
+            if ctx.needs_input_grad[0]:
+                gx = linear_grad_x(qweight, wscale, gy, kin, xdt)
+            if ctx.needs_input_grad[1]:
+                gw = linear_grad_w(q, a_scale, gy, kin, wdt)
+            if bdt is not None and ctx.needs_input_grad[2]:
+                gb = gy.to(torch.float32).sum(0).to(bdt)
+            return gx, gw, gb, None
+        g = gy.to(torch.float32).contiguous()
         if ctx.needs_input_grad[0]:
             w_deq = unpack_i2s(qweight)[:, :kin].to(torch.float32) * wscale  # [N, K]
             gx = (g @ w_deq).to(xdt)
@@ -117,16 +136,24 @@ class _SubLNBitLinearSTE(torch.autograd.Function):
     def backward(ctx, gy):
         x2, gamma, q, a_scale, qweight, wscale = ctx.saved_tensors
         wdt, bdt, kin, eps = ctx.meta
-        g = gy.to(torch.float32).contiguous()
+        kernels = _kernel_grads(gy, kin)
+        gy = gy.contiguous()
+        g = gy.to(torch.float32)
         gx = gg = gw = gb = None
         if ctx.needs_input_grad[2]:
-            x_deq = q[:, :kin].to(torch.float32) * a_scale[:, None]
-            gw = (g.t().contiguous() @ x_deq).to(wdt)
+            if kernels:
+                gw = linear_grad_w(q, a_scale, gy, kin, wdt)
+            else:
+                x_deq = q[:, :kin].to(torch.float32) * a_scale[:, None]
+                gw = (g.t().contiguous() @ x_deq).to(wdt)
         if bdt is not None and ctx.needs_input_grad[3]:
             gb = g.sum(0).to(bdt)
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            w_deq = unpack_i2s(qweight)[:, :kin].to(torch.float32) * wscale
-            g_norm = g @ w_deq  # gradient at the norm's output (identity through the quantiser)
+            # gradient at the norm's output (identity through the quantiser)
+            if kernels:
+                g_norm = linear_grad_x(qweight, wscale, gy, kin, torch.float32)
+            else:
+                g_norm = g @ (unpack_i2s(qweight)[:, :kin].to(torch.float32) * wscale)
             with torch.enable_grad():
                 xr = x2.detach().to(torch.float32).requires_grad_(ctx.needs_input_grad[0])
                 gr = gamma.detach().to(torch.float32).requires_grad_(ctx.needs_input_grad[1])

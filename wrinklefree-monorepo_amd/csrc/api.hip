@@ -199,6 +199,61 @@ int wfb_unpack_i2s(const uint8_t* qweight, int64_t n, int64_t k, int8_t* w_out, 
   return hip_status(wfb::launch_unpack_i2s(qweight, n, k, w_out, as_stream(stream)), "wfb_unpack_i2s");
 }
 
+namespace {
+// what both gradient entry points need of their sizes; the operand tiles are addressed through 32-bit offsets
+// from a tile's first row (256 rows of less than 2^20 elements)
+int grad_sizes(const char* name, int64_t m, int64_t n, int64_t k, int g_dtype) {
+  if (!valid_dtype(g_dtype)) return fail(WFB_EINVAL, "%s: bad gradient dtype %d", name, g_dtype);
+  constexpr int64_t kMax = (int64_t)1 << 20;
+  if (m < 1 || n < 1 || k < 1 || m >= kMax || n >= kMax || k >= kMax)
+    return fail(WFB_EINVAL, "%s: sizes m=%lld n=%lld k=%lld outside 1..2^20-1", name, (long long)m, (long long)n,
+                (long long)k);
+  return WFB_OK;
+}
+int grad_operands(const char* name, const void* g, int64_t ldg, int64_t n, const void* out, int out_dtype, int64_t ldo,
+                  int64_t k, const void* work) {
+  if (!g || !out || !work) return fail(WFB_EINVAL, "%s: null pointer", name);
+  if (!valid_dtype(out_dtype)) return fail(WFB_EINVAL, "%s: bad output dtype %d", name, out_dtype);
+  if (ldg < n || ldg >= (int64_t)1 << 21 || ldo < k)
+    return fail(WFB_EINVAL, "%s: row strides must satisfy N <= ldg < 2^21, ldo >= K", name);
+  if (!aligned(work, 16)) return fail(WFB_EINVAL, "%s: work must be 16-byte aligned", name);
+  return WFB_OK;
+}
+}  // namespace
+
+int wfb_linear_grad_workspace(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* bytes_x, int64_t* bytes_w) {
+  if (const int st = grad_sizes("wfb_linear_grad_workspace", m, n, k, g_dtype)) return st;
+  if (bytes_x) *bytes_x = wfb::grad_x_workspace(m, n, k, g_dtype);
+  if (bytes_w) *bytes_w = wfb::grad_w_workspace(m, n, k);
+  return ok();
+}
+
+int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const uint8_t* qweight, int64_t k,
+                      int64_t k_pad, const float* w_scale_dev, void* out, int out_dtype, int64_t ldo, void* work,
+                      void* stream) {
+  const char* name = "wfb_linear_grad_x";
+  if (const int st = grad_sizes(name, m, n, k, g_dtype)) return st;
+  if (const int st = grad_operands(name, g, ldg, n, out, out_dtype, ldo, k, work)) return st;
+  if (!qweight || !w_scale_dev) return fail(WFB_EINVAL, "%s: null pointer", name);
+  if (k_pad < k || k_pad % WFB_QK_I2S != 0 || !aligned(qweight, 8))
+    return fail(WFB_EINVAL, "%s: packed rows must be 8-byte aligned and hold k_pad >= K weights, a multiple of %d", name,
+                WFB_QK_I2S);
+  return hip_status(wfb::launch_grad_x(g, g_dtype, ldg, m, n, qweight, k, k_pad, w_scale_dev, out, out_dtype, ldo, work,
+                                       as_stream(stream)), name);
+}
+
+int wfb_linear_grad_w(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const int8_t* act, int64_t lda,
+                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* work,
+                      void* stream) {
+  const char* name = "wfb_linear_grad_w";
+  if (const int st = grad_sizes(name, m, n, k, g_dtype)) return st;
+  if (const int st = grad_operands(name, g, ldg, n, out, out_dtype, ldo, k, work)) return st;
+  if (!act || !a_scale) return fail(WFB_EINVAL, "%s: null pointer", name);
+  if (lda < k) return fail(WFB_EINVAL, "%s: activation row stride (%lld) < K (%lld)", name, (long long)lda, (long long)k);
+  return hip_status(wfb::launch_grad_w(g, g_dtype, ldg, m, n, act, lda, a_scale, k, out, out_dtype, ldo, work,
+                                       as_stream(stream)), name);
+}
+
 int wfb_quantize_act_i8(const void* x, int x_dtype, int64_t m, int64_t h, int64_t ldx, int8_t* q, int64_t k_pad,
                         int64_t ldq, float* a_scale, void* stream) {
   if (!valid_dtype(x_dtype)) return fail(WFB_EINVAL, "wfb_quantize_act_i8: bad dtype %d", x_dtype);

@@ -478,6 +478,14 @@ hipError_t launch_weight_absmean(const void* w, int dt, int64_t numel, float* sc
 hipError_t launch_pack_i2s(const void* w, int dt, int64_t n, int64_t k, int64_t ldw, const float* scale,
                            uint8_t* qw, hipStream_t s);
 hipError_t launch_unpack_i2s(const uint8_t* qw, int64_t n, int64_t k, int8_t* out, hipStream_t s);
+// Straight-through gradients (grad.hip); workspace bytes of each.
+int64_t grad_x_workspace(int64_t m, int64_t n, int64_t k, int gdt);
+int64_t grad_w_workspace(int64_t m, int64_t n, int64_t k);
+hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const uint8_t* qw, int64_t k,
+                         int64_t k_pad, const float* w_scale, void* out, int odt, int64_t ldo, void* work,
+                         hipStream_t s);
+hipError_t launch_grad_w(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const int8_t* q, int64_t ldq,
+                         const float* a_scale, int64_t k, void* out, int odt, int64_t ldo, void* work, hipStream_t s);
 hipError_t launch_quant_rows(const void* x, int dt, int64_t ldx, const void* gamma, int gdt, bool norm,
                              float eps, int64_t m, int64_t h, int8_t* q, int64_t k_pad, int64_t ldq,
                              float* a_scale, hipStream_t s);

@@ -641,6 +641,75 @@ def bitnet_linear_glu(
     return out
 
 
+# ---- gradients of the straight-through linear ------------------------------------------------------
+
+
+def linear_grad_supported(grad: torch.Tensor, in_features: int) -> bool:
+    """Whether linear_grad_x / linear_grad_w take this gradient [M, N]: a float tensor with memory of its own on a
+    HIP device (not one a functorch transform stands in for), no dimension empty, each below 2^20."""
+    if grad.device.type != "cuda" or grad.dtype not in _DT or grad.dim() != 2:
+        return False
+    m, n = grad.shape
+    if not (0 < m < 1 << 20 and 0 < n < 1 << 20 and 0 < in_features < 1 << 20):
+        return False
+    try:
+        grad.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
+def _grad_workspace(m: int, n: int, k: int, dt: int, which: int, dev: torch.device) -> torch.Tensor:
+    size = ctypes.c_int64(0)
+    ptr = ctypes.cast(ctypes.byref(size), ctypes.c_void_p)
+    _lib.call("wfb_linear_grad_workspace", m, n, k, dt, ptr if which == 0 else None, ptr if which == 1 else None)
+    return torch.empty(size.value, dtype=torch.uint8, device=dev)
+
+
+def linear_grad_x(packed_weights: torch.Tensor, scale: torch.Tensor, grad: torch.Tensor, in_features: int,
+                  out_dtype: torch.dtype) -> torch.Tensor:
+    """grad_x [M, in_features] = (grad @ ternary weight) * scale of a BitLinear's output gradient [M, N], in fp32 and
+    rounded once to ``out_dtype``; ``scale`` is the weight's fp32 device scalar."""
+    name = "linear_grad_x"
+    n, kb = packed_weights.shape
+    grad = grad.contiguous()
+    dev = _require_gpu(name, packed_weights, scale, grad)
+    if grad.dim() != 2 or grad.shape[1] != n or not 0 < in_features <= kb * 4:
+        raise RuntimeError(f"{name}: grad must be [tokens, {n}] and in_features at most {kb * 4}")
+    if scale.dtype != torch.float32 or scale.numel() != 1 or out_dtype not in _DT:
+        raise RuntimeError(f"{name}: scale must be one fp32 element and out_dtype a float type")
+    m, dt = grad.shape[0], _float_dtype(name, grad)
+    out = torch.empty((m, in_features), dtype=out_dtype, device=dev)
+    work = _grad_workspace(m, n, in_features, dt, 0, dev)
+    with torch.cuda.device(dev):
+        _lib.call("wfb_linear_grad_x", _p(grad), dt, n, m, n, _p(packed_weights), in_features, kb * 4, _p(scale),
+                  _p(out), _DT[out_dtype], in_features, _p(work), _stream(dev))
+    return out
+
+
+def linear_grad_w(codes: torch.Tensor, a_scale: torch.Tensor, grad: torch.Tensor, in_features: int,
+                  out_dtype: torch.dtype) -> torch.Tensor:
+    """grad_w [N, in_features] = (grad * a_scale)^T @ codes of a BitLinear's output gradient [M, N] and its int8
+    activation codes [M, k_pad] with per-token scales [M], in fp32 and rounded once to ``out_dtype``."""
+    name = "linear_grad_w"
+    grad = grad.contiguous()
+    dev = _require_gpu(name, a_scale, grad)
+    m, n = grad.shape
+    if codes.dtype != torch.int8 or codes.dim() != 2 or codes.shape[0] != m or codes.stride(1) != 1 \
+            or not 0 < in_features <= codes.shape[1] or codes.device != dev:
+        raise RuntimeError(f"{name}: codes must be int8 [{m}, >= in_features] with contiguous rows on {dev}")
+    if a_scale.dtype != torch.float32 or a_scale.numel() != m or out_dtype not in _DT:
+        raise RuntimeError(f"{name}: a_scale must be fp32 with one element per token and out_dtype a float type")
+    dt = _float_dtype(name, grad)
+    out = torch.empty((n, in_features), dtype=out_dtype, device=dev)
+    work = _grad_workspace(m, n, in_features, dt, 1, dev)
+    lda = codes.stride(0) if m > 1 else codes.shape[1]
+    with torch.cuda.device(dev):
+        _lib.call("wfb_linear_grad_w", _p(grad), dt, n, m, n, _p(codes), lda, _p(a_scale), in_features, _p(out),
+                  _DT[out_dtype], in_features, _p(work), _stream(dev))
+    return out
+
+
 # ---- greedy decoding: LM head + argmax ----------------------------------------------------------
 
 
