@@ -377,15 +377,25 @@ int wfb_linear_i2s_glu(const uint8_t* qweight, int64_t n, int64_t k, const int8_
  *   grad_w[n, k] = sum_m (g[m, n] * a_scale[m]) * act[m, k]             (wfb_linear_grad_w, act the int8 codes)
  * for k < K (K <= k_pad, the packed row length), in fp32: every product is exact, g * a_scale is rounded once to
  * fp32 and the sums are fp32.  g: fp32 / bf16 / fp16 [M, N], row stride ldg; w_scale_dev, a_scale: fp32 on the
- * device; out: fp32 / bf16 / fp16, row stride ldo.  work: 16-byte aligned device memory of at least the bytes
+ * device; out: fp32 / bf16 / fp16, row stride ldo.  bias_out [N] of type bias_dtype (or NULL) takes sum_m g[m, n],
+ * summed in fp32.  work: 16-byte aligned device memory of at least the bytes
  * wfb_linear_grad_workspace reports (host only, no GPU work).  M, N, K >= 1 and below 2^20 each. */
 int wfb_linear_grad_workspace(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* bytes_x, int64_t* bytes_w);
 int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const uint8_t* qweight,
                       int64_t k, int64_t k_pad, const float* w_scale_dev, void* out, int out_dtype, int64_t ldo,
                       void* work, void* stream);
 int wfb_linear_grad_w(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const int8_t* act, int64_t lda,
-                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* work,
-                      void* stream);
+                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* bias_out,
+                      int bias_dtype, void* work, void* stream);
+
+/* Backward of y = x * r * gamma, r = (mean(x^2) + eps)^(-1/2) (WF/models/subln.py:42-59), in fp32:
+ *   grad_x = r * (g * gamma) - x * r^3 * mean(g * gamma * x),  grad_gamma[h] = sum_m g * x * r.
+ * x [M, H] (contiguous, H a multiple of 8 up to WFB_NORM_MAX_H), gamma [H], g fp32 [M, H] 16-byte aligned; grad_x of
+ * x's type, 16-byte aligned, or NULL; grad_gamma of type ggamma_dtype or NULL.  work: with grad_gamma, 16-byte
+ * aligned, min(M, 512) * H floats. */
+int wfb_rmsnorm_grad(const void* x, int x_dtype, const void* gamma, int gamma_dtype, const float* g, float eps,
+                     int64_t m, int64_t h, void* grad_x, void* grad_gamma, int ggamma_dtype, float* work,
+                     void* stream);
 
 #ifdef __cplusplus
 }

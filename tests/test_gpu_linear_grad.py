@@ -72,3 +72,23 @@ def test_gradients_of_gradients_and_batched_gradients_keep_working(pkg, dev):
     both = torch.stack([gy.detach(), 2 * gy.detach()])
     bx, bw = torch.autograd.grad(mod(x), [x, mod.weight], both, is_grads_batched=True)
     assert _rel(bx[0], plain[0].double()) <= 1e-6 and _rel(bw[1], 2 * plain[1].double()) <= 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
+def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):
+    """Vector remainders of the 256-thread rows, more rows than workgroups, every row-length form.  fp32 sums of H
+    and of M terms: normwise error below 1e-6; 16-bit results are rounded once (2^-9 at most)."""
+    g = torch.Generator(device=dev).manual_seed(m + h)
+    x = torch.randn((m, h), generator=g, device=dev).to(dtype)
+    w = (1 + 0.1 * torch.randn(h, generator=g, device=dev)).to(dtype)
+    gy = torch.randn((m, h), generator=g, device=dev)
+    x64, w64 = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y = x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-6) * w64
+    want = torch.autograd.grad(y, [x64, w64], gy.double())
+    got = pkg.ops.rmsnorm_grad(x, w, gy, 1e-6)
+    tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for a, b in zip(got, want):
+        assert a.dtype == dtype and _rel(a, b) <= tol
+    only = pkg.ops.rmsnorm_grad(x, w, gy, 1e-6, need_x=False)
+    assert only[0] is None and torch.equal(only[1], got[1])

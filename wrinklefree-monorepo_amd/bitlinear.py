@@ -37,6 +37,7 @@ from .ops import (
     pack_ternary_i2s,
     quantize_activations_i8,
     quantize_activations_i8_per_token,
+    rmsnorm_grad,
     rmsnorm_quantize_i8,
     unpack_i2s,
 )
@@ -76,6 +77,16 @@ def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
     return not torch.is_grad_enabled() and linear_grad_supported(gy, in_features)
 
 
+def _weight_grads(q: torch.Tensor, a_scale: torch.Tensor, gy: torch.Tensor, kin: int, wdt: torch.dtype,
+                  bdt: Optional[torch.dtype], need_w: bool, need_b: bool):
+    """(grad_w or None, grad_b or None) on the gradient kernels; the bias sums ride in grad_w's operand pass."""
+    need_b = need_b and bdt is not None
+    if need_w and need_b:
+        return linear_grad_w(q, a_scale, gy, kin, wdt, bdt)
+    return (linear_grad_w(q, a_scale, gy, kin, wdt) if need_w else None,
+            gy.to(torch.float32).sum(0).to(bdt) if need_b else None)
+
+
 class _BitLinearSTE(torch.autograd.Function):
     """Straight-through estimator of the reference training forward at lambda = 1
     (WF/models/bitlinear.py:86-113).  Forward: the kernels' quantised product (per-token int8 codes of x,
@@ -100,10 +111,7 @@ class _BitLinearSTE(torch.autograd.Function):
             gy = gy.contiguous()
             if ctx.needs_input_grad[0]:
                 gx = linear_grad_x(qweight, wscale, gy, kin, xdt)
-            if ctx.needs_input_grad[1]:
-                gw = linear_grad_w(q, a_scale, gy, kin, wdt)
-            if bdt is not None and ctx.needs_input_grad[2]:
-                gb = gy.to(torch.float32).sum(0).to(bdt)
+            gw, gb = _weight_grads(q, a_scale, gy, kin, wdt, bdt, *ctx.needs_input_grad[1:3])
             return gx, gw, gb, None
         g = gy.to(torch.float32).contiguous()
         if ctx.needs_input_grad[0]:
@@ -136,24 +144,25 @@ class _SubLNBitLinearSTE(torch.autograd.Function):
     def backward(ctx, gy):
         x2, gamma, q, a_scale, qweight, wscale = ctx.saved_tensors
         wdt, bdt, kin, eps = ctx.meta
-        kernels = _kernel_grads(gy, kin)
-        gy = gy.contiguous()
-        g = gy.to(torch.float32)
+        if _kernel_grads(gy, kin):
+            gy = gy.contiguous()
+            gw, gb = _weight_grads(q, a_scale, gy, kin, wdt, bdt, *ctx.needs_input_grad[2:4])
+            gx = gg = None
+            if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
+                # gradient at the norm's output (identity through the quantiser), then the norm's own
+                g_norm = linear_grad_x(qweight, wscale, gy, kin, torch.float32)
+                gx, gg = rmsnorm_grad(x2.detach().contiguous(), gamma.detach().contiguous(), g_norm, eps, *ctx.needs_input_grad[:2])
+            return gx, gg, gw, gb, None, None
+        g = gy.to(torch.float32).contiguous()
         gx = gg = gw = gb = None
         if ctx.needs_input_grad[2]:
-            if kernels:
-                gw = linear_grad_w(q, a_scale, gy, kin, wdt)
-            else:
-                x_deq = q[:, :kin].to(torch.float32) * a_scale[:, None]
-                gw = (g.t().contiguous() @ x_deq).to(wdt)
+            x_deq = q[:, :kin].to(torch.float32) * a_scale[:, None]
+            gw = (g.t().contiguous() @ x_deq).to(wdt)
         if bdt is not None and ctx.needs_input_grad[3]:
             gb = g.sum(0).to(bdt)
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            # gradient at the norm's output (identity through the quantiser)
-            if kernels:
-                g_norm = linear_grad_x(qweight, wscale, gy, kin, torch.float32)
-            else:
-                g_norm = g @ (unpack_i2s(qweight)[:, :kin].to(torch.float32) * wscale)
+            w_deq = unpack_i2s(qweight)[:, :kin].to(torch.float32) * wscale
+            g_norm = g @ w_deq  # gradient at the norm's output (identity through the quantiser)
             with torch.enable_grad():
                 xr = x2.detach().to(torch.float32).requires_grad_(ctx.needs_input_grad[0])
                 gr = gamma.detach().to(torch.float32).requires_grad_(ctx.needs_input_grad[1])

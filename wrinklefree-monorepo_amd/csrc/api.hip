@@ -243,15 +243,33 @@ int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_
 }
 
 int wfb_linear_grad_w(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const int8_t* act, int64_t lda,
-                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* work,
-                      void* stream) {
+                      const float* a_scale, int64_t k, void* out, int out_dtype, int64_t ldo, void* bias_out,
+                      int bias_dtype, void* work, void* stream) {
   const char* name = "wfb_linear_grad_w";
   if (const int st = grad_sizes(name, m, n, k, g_dtype)) return st;
   if (const int st = grad_operands(name, g, ldg, n, out, out_dtype, ldo, k, work)) return st;
   if (!act || !a_scale) return fail(WFB_EINVAL, "%s: null pointer", name);
   if (lda < k) return fail(WFB_EINVAL, "%s: activation row stride (%lld) < K (%lld)", name, (long long)lda, (long long)k);
-  return hip_status(wfb::launch_grad_w(g, g_dtype, ldg, m, n, act, lda, a_scale, k, out, out_dtype, ldo, work,
-                                       as_stream(stream)), name);
+  if (bias_out && !valid_dtype(bias_dtype)) return fail(WFB_EINVAL, "%s: bad bias dtype %d", name, bias_dtype);
+  return hip_status(wfb::launch_grad_w(g, g_dtype, ldg, m, n, act, lda, a_scale, k, out, out_dtype, ldo, bias_out,
+                                       bias_dtype, work, as_stream(stream)), name);
+}
+
+int wfb_rmsnorm_grad(const void* x, int x_dtype, const void* gamma, int gamma_dtype, const float* g, float eps,
+                     int64_t m, int64_t h, void* grad_x, void* grad_gamma, int ggamma_dtype, float* work,
+                     void* stream) {
+  const char* name = "wfb_rmsnorm_grad";
+  if (!valid_dtype(x_dtype) || !valid_dtype(gamma_dtype) || (grad_gamma && !valid_dtype(ggamma_dtype)))
+    return fail(WFB_EINVAL, "%s: bad dtype", name);
+  if (m < 0 || m > INT32_MAX / 2 || h <= 0 || h > WFB_NORM_MAX_H || h % 8 != 0)
+    return fail(WFB_EINVAL, "%s: H (%lld) must be a multiple of 8 in 8..%d", name, (long long)h, WFB_NORM_MAX_H);
+  if (m == 0) return ok();
+  if (!x || !gamma || !g || (!grad_x && !grad_gamma) || (grad_gamma && !work))
+    return fail(WFB_EINVAL, "%s: null pointer", name);
+  if (!aligned(g, 16) || !aligned(grad_x, 16) || !aligned(work, 16))
+    return fail(WFB_EINVAL, "%s: g, grad_x and work must be 16-byte aligned", name);
+  return hip_status(wfb::launch_norm_grad(x, x_dtype, gamma, gamma_dtype, g, eps, m, h, grad_x, grad_gamma,
+                                          ggamma_dtype, work, as_stream(stream)), name);
 }
 
 int wfb_quantize_act_i8(const void* x, int x_dtype, int64_t m, int64_t h, int64_t ldx, int8_t* q, int64_t k_pad,

@@ -47,25 +47,31 @@ __device__ __forceinline__ void split3(float v, uint16_t (&p)[3]) {
 
 // Planes of v[n][m] = g[m][n] * a_scale[m], dst[p][n][m] with rows of mp elements (m >= M: zeros).  One 64 x 64
 // tile per workgroup through LDS: whole 128-byte lines in and out; the padded rows keep both sides of the
-// transpose free of bank conflicts.
+// transpose free of bank conflicts.  With colsum, also the tile's column sums of g, colsum[m0 / 64][n].
 template <int DT>
 __global__ __launch_bounds__(256) void grad_scaled_t_kernel(const void* __restrict__ g, int64_t ldg,
                                                             const float* __restrict__ a_scale, int64_t M, int64_t N,
-                                                            int64_t mp, uint16_t* __restrict__ dst) {
+                                                            int64_t mp, uint16_t* __restrict__ dst,
+                                                            float* __restrict__ colsum) {
   __shared__ float tile[64][65];
+  __shared__ float sums[4][64];
   const int64_t m0 = (int64_t)blockIdx.x * 64, n0 = (int64_t)blockIdx.y * 64;
   const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
-  float v[16];
+  float v[16], sum = 0.0f;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int64_t m = m0 + r0 + 4 * j, n = n0 + c;
     const int64_t mc = m < M ? m : M - 1, nc = n < N ? n : N - 1;
     const float x = load_elem<DT>(g, mc * ldg + nc), s = a_scale[mc];
     v[j] = m < M ? __fmul_rn(x, s) : 0.0f;
+    sum += m < M ? x : 0.0f;
   }
+  sums[r0][c] = sum;
 #pragma unroll
   for (int j = 0; j < 16; ++j) tile[r0 + 4 * j][c] = v[j];
   __syncthreads();
+  if (colsum && r0 == 0 && n0 + c < N)
+    colsum[(int64_t)blockIdx.x * N + n0 + c] = (sums[0][c] + sums[1][c]) + (sums[2][c] + sums[3][c]);
   const int64_t plane = N * mp;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -522,7 +528,8 @@ int64_t grad_x_workspace(int64_t m, int64_t n, int64_t k, int gdt) {
 
 int64_t grad_w_workspace(int64_t m, int64_t n, int64_t k) {
   const int64_t mp = pad_to(m, kPad);
-  return align256(2 * 3 * n * mp) + align256(2 * k * mp) + part_bytes(plan(3, n, k, m), n, k);
+  return align256(2 * 3 * n * mp) + align256(2 * k * mp) + align256(4 * (mp / 64) * n) +
+         part_bytes(plan(3, n, k, m), n, k);
 }
 
 hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const uint8_t* qw, int64_t k,
@@ -569,21 +576,25 @@ hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t
 }
 
 hipError_t launch_grad_w(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const int8_t* q, int64_t ldq,
-                         const float* a_scale, int64_t k, void* out, int odt, int64_t ldo, void* work, hipStream_t s) {
+                         const float* a_scale, int64_t k, void* out, int odt, int64_t ldo, void* bias_out, int bdt,
+                         void* work, hipStream_t s) {
   const int64_t mp = pad_to(m, kPad);
   char* ws = static_cast<char*>(work);
   uint16_t* gt = reinterpret_cast<uint16_t*>(ws);
   uint16_t* qt = reinterpret_cast<uint16_t*>(ws + align256(2 * 3 * n * mp));
-  float* parts = reinterpret_cast<float*>(ws + align256(2 * 3 * n * mp) + align256(2 * k * mp));
+  float* sums = reinterpret_cast<float*>(ws + align256(2 * 3 * n * mp) + align256(2 * k * mp));
+  float* parts = reinterpret_cast<float*>(reinterpret_cast<char*>(sums) + align256(4 * (mp / 64) * n));
+  float* cs = bias_out ? sums : nullptr;
   const dim3 gg((unsigned)(mp / 64), (unsigned)((n + 63) / 64));
   if (gdt == WFB_F32)
-    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_F32>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt);
+    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_F32>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt, cs);
   else if (gdt == WFB_BF16)
-    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_BF16>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt);
+    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_BF16>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt, cs);
   else
-    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_F16>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt);
+    hipLaunchKernelGGL((grad_scaled_t_kernel<WFB_F16>), gg, dim3(256), 0, s, g, ldg, a_scale, m, n, mp, gt, cs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (bias_out && (e = launch_column_sum(sums, (int)(mp / 64), n, bias_out, bdt, s)) != hipSuccess) return e;
   const dim3 gq((unsigned)(mp / 64), (unsigned)((k + 63) / 64));
   if ((uintptr_t)q % 16 == 0 && ldq % 16 == 0)
     hipLaunchKernelGGL((codes_t_kernel<true>), gq, dim3(256), 0, s, q, ldq, m, k, mp, qt);

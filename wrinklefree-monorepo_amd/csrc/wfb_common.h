@@ -485,7 +485,13 @@ hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t
                          int64_t k_pad, const float* w_scale, void* out, int odt, int64_t ldo, void* work,
                          hipStream_t s);
 hipError_t launch_grad_w(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const int8_t* q, int64_t ldq,
-                         const float* a_scale, int64_t k, void* out, int odt, int64_t ldo, void* work, hipStream_t s);
+                         const float* a_scale, int64_t k, void* out, int odt, int64_t ldo, void* bias_out, int bdt,
+                         void* work, hipStream_t s);
+// RMSNorm backward (norm_grad.hip); part: norm_grad_parts(m) x h floats, needed with gw.
+int norm_grad_parts(int64_t m);
+hipError_t launch_norm_grad(const void* x, int dt, const void* w, int wdt, const float* g, float eps, int64_t m,
+                            int64_t h, void* gx, void* gw, int gw_dtype, float* part, hipStream_t s);
+hipError_t launch_column_sum(const float* part, int rows, int64_t cols, void* out, int out_dtype, hipStream_t s);
 hipError_t launch_quant_rows(const void* x, int dt, int64_t ldx, const void* gamma, int gdt, bool norm,
                              float eps, int64_t m, int64_t h, int8_t* q, int64_t k_pad, int64_t ldq,
                              float* a_scale, hipStream_t s);

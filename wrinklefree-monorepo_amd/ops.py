@@ -688,9 +688,10 @@ def linear_grad_x(packed_weights: torch.Tensor, scale: torch.Tensor, grad: torch
 
 
 def linear_grad_w(codes: torch.Tensor, a_scale: torch.Tensor, grad: torch.Tensor, in_features: int,
-                  out_dtype: torch.dtype) -> torch.Tensor:
+                  out_dtype: torch.dtype, bias_dtype: Optional[torch.dtype] = None):
     """grad_w [N, in_features] = (grad * a_scale)^T @ codes of a BitLinear's output gradient [M, N] and its int8
-    activation codes [M, k_pad] with per-token scales [M], in fp32 and rounded once to ``out_dtype``."""
+    activation codes [M, k_pad] with per-token scales [M], in fp32 and rounded once to ``out_dtype``.  With
+    ``bias_dtype`` also the bias gradient [N], grad summed over the tokens: (grad_w, grad_bias)."""
     name = "linear_grad_w"
     grad = grad.contiguous()
     dev = _require_gpu(name, a_scale, grad)
@@ -698,16 +699,37 @@ def linear_grad_w(codes: torch.Tensor, a_scale: torch.Tensor, grad: torch.Tensor
     if codes.dtype != torch.int8 or codes.dim() != 2 or codes.shape[0] != m or codes.stride(1) != 1 \
             or not 0 < in_features <= codes.shape[1] or codes.device != dev:
         raise RuntimeError(f"{name}: codes must be int8 [{m}, >= in_features] with contiguous rows on {dev}")
-    if a_scale.dtype != torch.float32 or a_scale.numel() != m or out_dtype not in _DT:
-        raise RuntimeError(f"{name}: a_scale must be fp32 with one element per token and out_dtype a float type")
+    if a_scale.dtype != torch.float32 or a_scale.numel() != m or out_dtype not in _DT \
+            or not (bias_dtype is None or bias_dtype in _DT):
+        raise RuntimeError(f"{name}: a_scale must be fp32 with one element per token and the outputs float types")
     dt = _float_dtype(name, grad)
     out = torch.empty((n, in_features), dtype=out_dtype, device=dev)
+    bias = None if bias_dtype is None else torch.empty(n, dtype=bias_dtype, device=dev)
     work = _grad_workspace(m, n, in_features, dt, 1, dev)
     lda = codes.stride(0) if m > 1 else codes.shape[1]
     with torch.cuda.device(dev):
         _lib.call("wfb_linear_grad_w", _p(grad), dt, n, m, n, _p(codes), lda, _p(a_scale), in_features, _p(out),
-                  _DT[out_dtype], in_features, _p(work), _stream(dev))
-    return out
+                  _DT[out_dtype], in_features, _p(bias), _DT[bias_dtype] if bias is not None else 0, _p(work),
+                  _stream(dev))
+    return out if bias is None else (out, bias)
+
+
+def rmsnorm_grad(x: torch.Tensor, weight: torch.Tensor, grad: torch.Tensor, eps: float, need_x: bool = True,
+                 need_weight: bool = True):
+    """(grad_x or None, grad_weight or None) of y = x * rsqrt(mean(x^2) + eps) * weight for x [M, H] and the fp32
+    gradient [M, H] at y, in fp32 and rounded once to the inputs' types."""
+    name = "rmsnorm_grad"
+    dev = _require_gpu(name, x, weight, grad)
+    m, h = x.shape
+    if grad.dtype != torch.float32 or grad.shape != x.shape or weight.numel() != h:
+        raise RuntimeError(f"{name}: grad must be float32 {list(x.shape)} and weight have {h} elements")
+    gx = torch.empty_like(x) if need_x else None
+    gw = torch.empty_like(weight) if need_weight else None
+    work = torch.empty(min(m, 512) * h, dtype=torch.float32, device=dev) if need_weight else None
+    with torch.cuda.device(dev):
+        _lib.call("wfb_rmsnorm_grad", _p(x), _float_dtype(name, x), _p(weight), _float_dtype(name, weight), _p(grad),
+                  float(eps), m, h, _p(gx), _p(gw), _DT[weight.dtype], _p(work), _stream(dev))
+    return gx, gw
 
 
 # ---- greedy decoding: LM head + argmax ----------------------------------------------------------
