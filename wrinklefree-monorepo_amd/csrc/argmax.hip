@@ -14,7 +14,14 @@
 // RMSNorm of the M token rows (y = x * (1/sqrt(mean(x^2) + eps)) * gamma, rounded to the x dtype as the
 // torch glue does) into LDS, then streams 64 vocabulary rows: 8 lanes per row, each lane a 16-byte
 // (bf16) or 32-byte (fp32) piece of the row per step against the normalised rows in LDS, fp32
-// accumulation, a DPP sum over the 8 lanes; each wave covers 16 rows = one workspace slot.
+// accumulation, a DPP sum over the 8 lanes; each wave covers 16 rows = one workspace slot.  bf16 rows against a
+// bf16 embedding (the normalised rows are bf16 values then) are kept as bf16 in LDS and multiplied two elements per
+// instruction (v_dot2c_f32_bf16, exact products, fp32 sums), and from two tokens on each LDS read serves a wave's two
+// groups of 8 rows.  One token is bound by the weight stream; at more, widening, multiplying and adding each element
+// of each token by itself took 9 vector operations a weight at 4 tokens, and the rows twice the LDS bytes.  Whole
+// call with the finalize, before and after: 128256 x 2560 at M = 2 134 -> 119 us, M = 4 174 -> 131 (5.0 TB/s), M = 6
+// 262 -> 143; 128256 x 1024 at M = 16 255 -> 136; 49152 x 576 at M = 8 38 -> 31; M = 1 unchanged (its two row
+// groups stay one after the other: together they took 66 instead of 56 us at 33333 x 4096).
 #include "wfb_common.h"
 
 namespace wfb {
@@ -74,7 +81,9 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x
                                                       const void* __restrict__ W, int64_t ldw, int m, int n, int h,
                                                       float* __restrict__ logits, int64_t ldo,
                                                       uint64_t* __restrict__ parts) {
-  extern __shared__ float xn[];  // [m][h]
+  constexpr bool DOT = XT == WFB_BF16 && WT == WFB_BF16;
+  extern __shared__ float xn[];  // [m][h], as bf16 with DOT
+  uint16_t* const xh = reinterpret_cast<uint16_t*>(xn);
   __shared__ float rs[16];
   __shared__ float red[4][MM];
   constexpr int ESZ = WT == WFB_F32 ? 4 : 2;
@@ -153,13 +162,19 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x
       const int i = (j0 + u) * 256 + t;
       if (i >= nch) break;
       const int mm = i / C8, c = i - mm * C8;
+      uint32_t hw[4] = {0, 0, 0, 0};
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float y = v[u][e] * rs[mm];
         if (gamma) y = y * gv[u][e];
-        if constexpr (XT == WFB_BF16) y = bf16_bits_to_f32(f32_to_bf16_rne(y));
-        xn[mm * h + 8 * c + e] = y;
+        if constexpr (DOT) {
+          hw[e / 2] |= (uint32_t)f32_to_bf16_rne(y) << (16 * (e & 1));
+        } else {
+          if constexpr (XT == WFB_BF16) y = bf16_bits_to_f32(f32_to_bf16_rne(y));
+          xn[mm * h + 8 * c + e] = y;
+        }
       }
+      if constexpr (DOT) *reinterpret_cast<uint4*>(xh + mm * h + 8 * c) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
     }
   }
   __syncthreads();
@@ -169,54 +184,8 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x
   uint64_t best[MM];
 #pragma unroll
   for (int mm = 0; mm < MM; ++mm) best[mm] = 0;
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const int row = blockIdx.x * 64 + w * 16 + p * 8 + rsub;
-    const uint32_t roff = (uint32_t)((int64_t)row * ldw * ESZ);
-    float acc[MM];
-#pragma unroll
-    for (int mm = 0; mm < MM; ++mm) acc[mm] = 0.0f;
-    // U chunks' loads in flight per lane, then their arithmetic in chunk order (a one-load-then-wait loop
-    // kept a single 16-byte load in flight per lane); chunks past the row read zeros from an out-of-range
-    // offset (below 2^31, so offset + 16 cannot wrap) and add exactly +0
-    constexpr int U = 4;
-    for (int c0 = s; c0 < C; c0 += 8 * U) {
-      v4i r0[U], r1[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int c = c0 + 8 * u;
-        const uint32_t off = c < C ? roff + (uint32_t)(8 * c * ESZ) : 0x7FFFFF00u;
-        r0[u] = buf_load16(wb, off);
-        if constexpr (WT == WFB_F32) r1[u] = buf_load16(wb, off + 16);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int c = c0 + 8 * u < C ? c0 + 8 * u : 0;  // the LDS index stays in range (its weights are 0)
-        float wv[8];
-        if constexpr (WT == WFB_F32) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            wv[e] = __int_as_float(r0[u][e]);
-            wv[4 + e] = __int_as_float(r1[u][e]);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            wv[2 * e] = __uint_as_float((uint32_t)r0[u][e] << 16);
-            wv[2 * e + 1] = __uint_as_float((uint32_t)r0[u][e] & 0xffff0000u);
-          }
-        }
-#pragma unroll
-        for (int mm = 0; mm < MM; ++mm) {
-          if (mm < m) {
-            const float4* xp = reinterpret_cast<const float4*>(xn + mm * h + 8 * c);
-            const float4 a = xp[0], b = xp[1];
-            acc[mm] += wv[0] * a.x + wv[1] * a.y + wv[2] * a.z + wv[3] * a.w + wv[4] * b.x + wv[5] * b.y +
-                       wv[6] * b.z + wv[7] * b.w;
-          }
-        }
-      }
-    }
+  // logit of (token mm, row) from the 8 lanes' sums: stored, and its key taken into the wave's best
+  auto finish = [&](int row, const float (&acc)[MM]) {
     const bool valid = row < n && s == 0;
 #pragma unroll
     for (int mm = 0; mm < MM; ++mm) {
@@ -226,6 +195,103 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x
         const uint64_t key = group_max_u64<64>(valid ? amax_key(y, row) : 0);
         best[mm] = key > best[mm] ? key : best[mm];
       }
+    }
+  };
+  // U chunks' loads in flight per lane (and row group), then their arithmetic in chunk order (a one-load-then-wait
+  // loop kept a single 16-byte load in flight per lane); chunks past the row read zeros from an out-of-range
+  // offset (below 2^31, so offset + 16 cannot wrap) and add exactly +0
+  constexpr int U = 4;
+  const int row0 = blockIdx.x * 64 + w * 16 + rsub;
+  if constexpr (DOT) {
+    constexpr int NP = MM == 1 ? 1 : 2;  // row groups at once
+#pragma unroll
+    for (int p0 = 0; p0 < 2; p0 += NP) {
+      float acc[NP][MM];
+      uint32_t roff[NP];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        roff[p] = (uint32_t)((int64_t)(row0 + 8 * (p0 + p)) * ldw * ESZ);
+#pragma unroll
+        for (int mm = 0; mm < MM; ++mm) acc[p][mm] = 0.0f;
+      }
+      for (int c0 = s; c0 < C; c0 += 8 * U) {
+        v4i r[NP][U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            const int c = c0 + 8 * u;
+            r[p][u] = buf_load16(wb, c < C ? roff[p] + (uint32_t)(16 * c) : 0x7FFFFF00u);
+          }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + 8 * u < C ? c0 + 8 * u : 0;  // the LDS index stays in range (its weights are 0)
+#pragma unroll
+          for (int mm = 0; mm < MM; ++mm) {
+            if (mm < m) {
+              const v4i y = *reinterpret_cast<const v4i*>(xh + mm * h + 8 * c);
+#pragma unroll
+              for (int p = 0; p < NP; ++p) {
+                float d = 0.0f;  // a chunk's own sum first: one rounding at the running sum's size per 8 elements
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  d = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, (int)r[p][u][e]),
+                                                      __builtin_bit_cast(bf16x2_t, (int)y[e]), d, false);
+                acc[p][mm] += d;
+              }
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < NP; ++p) finish(row0 + 8 * (p0 + p), acc[p]);
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int row = row0 + 8 * p;
+      const uint32_t roff = (uint32_t)((int64_t)row * ldw * ESZ);
+      float acc[MM];
+#pragma unroll
+      for (int mm = 0; mm < MM; ++mm) acc[mm] = 0.0f;
+      for (int c0 = s; c0 < C; c0 += 8 * U) {
+        v4i r0[U], r1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + 8 * u;
+          const uint32_t off = c < C ? roff + (uint32_t)(8 * c * ESZ) : 0x7FFFFF00u;
+          r0[u] = buf_load16(wb, off);
+          if constexpr (WT == WFB_F32) r1[u] = buf_load16(wb, off + 16);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + 8 * u < C ? c0 + 8 * u : 0;  // the LDS index stays in range (its weights are 0)
+          float wv[8];
+          if constexpr (WT == WFB_F32) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              wv[e] = __int_as_float(r0[u][e]);
+              wv[4 + e] = __int_as_float(r1[u][e]);
+            }
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              wv[2 * e] = __uint_as_float((uint32_t)r0[u][e] << 16);
+              wv[2 * e + 1] = __uint_as_float((uint32_t)r0[u][e] & 0xffff0000u);
+            }
+          }
+#pragma unroll
+          for (int mm = 0; mm < MM; ++mm) {
+            if (mm < m) {
+              const float4* xp = reinterpret_cast<const float4*>(xn + mm * h + 8 * c);
+              const float4 a = xp[0], b = xp[1];
+              acc[mm] += wv[0] * a.x + wv[1] * a.y + wv[2] * a.z + wv[3] * a.w + wv[4] * b.x + wv[5] * b.y +
+                         wv[6] * b.z + wv[7] * b.w;
+            }
+          }
+        }
+      }
+      finish(row, acc);
     }
   }
   const int slot = blockIdx.x * 4 + w;
@@ -240,7 +306,7 @@ template <int XT, int WT>
 hipError_t launch_head_t(const void* x, int64_t ldx, const void* gamma, int gdt, float eps, const void* w, int64_t ldw,
                          int m, int n, int h, float* logits, int64_t ldo, uint64_t* parts, hipStream_t s) {
   const dim3 grid((n + 63) / 64);
-  const size_t lds = (size_t)m * h * sizeof(float);
+  const size_t lds = (size_t)m * h * (XT == WFB_BF16 && WT == WFB_BF16 ? 2 : 4);
 #define WFB_HEAD(MMV) \
   hipLaunchKernelGGL((lm_head_kernel<XT, WT, MMV>), grid, dim3(256), lds, s, x, ldx, gamma, gdt, eps, w, ldw, m, n, h, \
                      logits, ldo, parts)
