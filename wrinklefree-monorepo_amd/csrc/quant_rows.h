@@ -131,9 +131,9 @@ __device__ __forceinline__ buf_t row_buf(const void* r, int h) {
   return make_buf(r, (uint32_t)h * (DT == WFB_F32 ? 4u : 2u));
 }
 
-// IT: vectors per thread the row can need, kMaxIt or half of it.  Rows up to 8192 take the half: the vectors they do
-// not have cost registers (140 against 76: 3 waves per SIMD instead of 6) and as many serial zero additions as the
-// row's own.  8192 x 6912 bf16 with gamma: 61 -> 39 us (4.3 TB/s), traced.
+// IT: vectors per thread that the row needs.  Vectors it does not have would cost registers (76 at IT = 4, 140 at
+// the longest rows' 8: 6 waves per SIMD instead of 3) and serial zero additions.  With 8 for every row, 8192 x 6912
+// bf16 with gamma took 61 us, with its own 4 39 us (4.3 TB/s); 8 rows of 14336 fp32 7.7 us, with 7 7.3 (traced).
 template <int DT, int GDT, bool NORM, int GLU, int IT>
 __global__ __launch_bounds__(kTPB) void quant_rows_kernel(const void* __restrict__ x, const void* __restrict__ up,
                                                           int64_t ldx, const void* __restrict__ gamma, float eps,
@@ -543,12 +543,20 @@ hipError_t launch_rows_t(const void* x, const void* up, int64_t ldx, const void*
       case 9: case 10: case 11: case 12: WFB_WAVE(12); break;
       default: WFB_WAVE(16); break;
     }
-  } else if (h <= kTPB * kVec * kMaxIt / 2) {
-    hipLaunchKernelGGL((quant_rows_kernel<DT, GDT, NORM, GLU, kMaxIt / 2>), dim3((unsigned)m), dim3(kTPB), 0, s, x, up,
-                       ldx, gamma, eps, (int)h, q, k_pad, ldq, a_scale, vec);
   } else {
-    hipLaunchKernelGGL((quant_rows_kernel<DT, GDT, NORM, GLU, kMaxIt>), dim3((unsigned)m), dim3(kTPB), 0, s, x, up, ldx,
-                       gamma, eps, (int)h, q, k_pad, ldq, a_scale, vec);
+#define WFB_ROWS(I)                                                                                                 \
+  hipLaunchKernelGGL((quant_rows_kernel<DT, GDT, NORM, GLU, I>), dim3((unsigned)m), dim3(kTPB), 0, s, x, up, ldx, gamma, \
+                     eps, (int)h, q, k_pad, ldq, a_scale, vec)
+    static_assert(kWaveMaxH == 2 * kTPB * kVec && kMaxIt == 8, "vectors per thread of the longer rows: 3 .. 8");
+    switch ((int)((h + kTPB * kVec - 1) / (kTPB * kVec))) {
+      case 3: WFB_ROWS(3); break;
+      case 4: WFB_ROWS(4); break;
+      case 5: WFB_ROWS(5); break;
+      case 6: WFB_ROWS(6); break;
+      case 7: WFB_ROWS(7); break;
+      default: WFB_ROWS(8); break;
+    }
+#undef WFB_ROWS
   }
 #undef WFB_WAVE
   return hipGetLastError();
