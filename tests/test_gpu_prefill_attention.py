@@ -157,3 +157,27 @@ def test_prefill_attention_python_errors(pkg, dev):
         pkg.gqa_prefill_attention(q, kv, kv, kc, kc.clone(), 30, 4)
     with pytest.raises(RuntimeError, match="rope"):
         pkg.gqa_prefill_attention(q, kv, kv, kc, kc.clone(), 0, 4, torch.zeros((32, 32), device=dev), None)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("g,t,start,scale", [(1, 33, 0, 0.1), (1, 129, 5, -0.1), (2, 65, 64, 0.09), (3, 32, 31, 0.0),
+                                             (4, 63, 100, 0.125), (4, 97, 0, 2.0), (5, 64, 1, 0.1), (6, 31, 33, 0.1),
+                                             (7, 33, 63, -1.0), (8, 70, 0, 0.1)])
+def test_many_workgroups_take_the_32_token_form(pkg, dev, d, g, t, start, scale):
+    """More than 256 blocks of 16 tokens, the line to the 32-token kernel: its query-block and key-block edges, every
+    group size, negative, zero and large scales (a large one moves the softmax reference between key blocks)."""
+    hkv, max_len = 2, start + t + 3
+    b = 257 * 16 // (t * hkv) + 1
+    gen = torch.Generator().manual_seed(100 * g + t)
+    q = torch.randn((b * t, hkv * g * d), generator=gen).to(torch.bfloat16)
+    k_new, v_new = (torch.randn((b * t, hkv * d), generator=gen).to(torch.bfloat16) for _ in range(2))
+    kc, vc = (torch.randn((b, hkv, max_len, d), generator=gen).to(torch.bfloat16) for _ in range(2))
+    kc[:, :, start + t:], vc[:, :, start + t:] = float("inf"), float("nan")  # must not leak in
+    cos, sin = _tables(max_len, d)
+    ref, kc_ref, vc_ref = _reference(q, k_new, v_new, kc, vc, start, t, cos, sin, hkv * g, scale)
+    kc_d, vc_d = kc.to(dev), vc.to(dev)
+    out = pkg.gqa_prefill_attention(q.to(dev), k_new.to(dev), v_new.to(dev), kc_d, vc_d, start, t, cos.to(dev),
+                                    sin.to(dev), scale=scale)
+    assert torch.equal(kc_d.cpu(), kc_ref) and torch.equal(vc_d.cpu().view(torch.int16), vc_ref.view(torch.int16))
+    err = (out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-2)
+    assert float(err.max()) <= 1e-2 and float(err.mean()) <= 2e-3
