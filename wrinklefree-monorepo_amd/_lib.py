@@ -71,6 +71,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_entry: dict = {}  # entry points by name, filled by load()
 _load_error: str | None = None
 
 
@@ -95,6 +96,7 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = ctypes.c_int
         fn.argtypes = argtypes
+        _entry[name] = fn
     _lib = lib
     return lib
 
@@ -113,10 +115,10 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Call an entry point; a non-zero status raises RuntimeError carrying wfb_last_error()."""
-    lib = load()
-    st = getattr(lib, name)(*args)
+    fn = _entry.get(name) or getattr(load(), name)
+    st = fn(*args)
     if st != WFB_OK:
-        raise RuntimeError(f"{name} failed ({st}): {lib.wfb_last_error().decode()}")
+        raise RuntimeError(f"{name} failed ({st}): {last_error()}")
 
 
 def status(name: str, *args) -> int:

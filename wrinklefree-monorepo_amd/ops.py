@@ -15,6 +15,7 @@ The ops are also registered as ``torch.ops.wfbitnet.*`` with the reference schem
 from __future__ import annotations
 
 import collections
+import contextlib
 import ctypes
 import weakref
 from typing import Optional, Sequence, Tuple, Union
@@ -37,29 +38,44 @@ def check_kernel_available() -> bool:
     return _lib.available() and torch.cuda.is_available()
 
 
-def _p(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+# What every call pays on the host.  A small call is bound by it, not by its kernels: one token through a 576 x 576
+# BitLinear is two launches, 30.2 us a call with a device guard, a stream object and pointer boxes around each and
+# 22.2 without (the fused MLP of one token 45.2 -> 32.7).  Pointers and streams go to the C entry points as plain
+# integers (their argument types are declared), the stream comes from torch's raw accessor, and the device guard is
+# entered only for a device that is not the current one.
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _p(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
+
+
+def _stream(dev: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """Context in which ``dev`` is the current device."""
+    return _HERE if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)
 
 
 def _require_gpu(name: str, *ts: Optional[torch.Tensor]) -> torch.device:
-    dev = None
+    first = None
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(f"{name}: tensors must be on a HIP device (got {t.device})")
         if not t.is_contiguous():
             raise RuntimeError(f"{name}: tensors must be contiguous")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"{name}: tensors are on different devices ({dev}, {t.device})")
-    assert dev is not None
-    return dev
+        if first is None:
+            first = t
+        elif t.get_device() != first.get_device():
+            raise RuntimeError(f"{name}: tensors are on different devices ({first.device}, {t.device})")
+    assert first is not None
+    return first.device
 
 
 def _float_dtype(name: str, t: torch.Tensor) -> int:
@@ -87,7 +103,7 @@ def absmean_scale(weights: torch.Tensor) -> torch.Tensor:
     dt = _float_dtype(name, weights)
     scale = torch.empty(1, dtype=torch.float32, device=dev)
     ws = torch.empty(WFB_ABSMEAN_WS_DOUBLES, dtype=torch.float64, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_weight_absmean", _p(weights), dt, weights.numel(), _p(scale), _p(ws), _stream(dev))
     return scale
 
@@ -119,7 +135,7 @@ def pack_ternary_i2s(
         w = torch.zeros((n, kp), dtype=weights.dtype, device=dev)
         w[:, :k] = weights
     packed = torch.empty((n, kp // 4), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_pack_i2s", _p(w), _DT[w.dtype], n, kp, kp, _p(scale.contiguous()), _p(packed), _stream(dev))
     return packed, scale
 
@@ -132,7 +148,7 @@ def unpack_i2s(packed_weights: torch.Tensor) -> torch.Tensor:
     dev = _require_gpu(name, packed_weights)
     n, kb = packed_weights.shape
     out = torch.empty((n, kb * 4), dtype=torch.int8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_unpack_i2s", _p(packed_weights), n, kb * 4, _p(out), _stream(dev))
     return out
 
@@ -172,7 +188,7 @@ def convert_hf_offline_i2s(
     qweight = torch.empty((n, kp // 4), dtype=torch.uint8, device=dev)
     scale = torch.empty(1, dtype=torch.float32, device=dev)
     work = torch.empty((n * (kp // 16) + 255) // 256 + 1, dtype=torch.int64, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_convert_hf_offline_i2s", _p(packed_hf), nb, n, k, kp, ws_ptr, ws_dt, ws_host,
                   _SCALE_MODES[scale_mode], _p(qweight), _p(scale), _p(work), _stream(dev))
     return qweight, scale
@@ -192,7 +208,7 @@ def quantize_activations_i8(activations: torch.Tensor) -> Tuple[torch.Tensor, to
     dt = _float_dtype(name, activations)
     q = torch.empty(activations.shape, dtype=torch.int8, device=dev)
     scale = torch.empty(1, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_quantize_act_i8_tensor", _p(activations), dt, activations.numel(), _p(q), _p(scale), _stream(dev))
     return q, scale
 
@@ -223,7 +239,7 @@ def quantize_activations_i8_per_token(
     h, kp, kpa, m = _rows(name, x, k_pad)
     q = torch.empty((*x.shape[:-1], kpa), dtype=torch.int8, device=dev)
     a_scale = torch.empty(x.shape[:-1], dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_quantize_act_i8", _p(x), dt, m, h, h, _p(q), kpa, kpa, _p(a_scale), _stream(dev))
     return (q if kpa == kp else q[..., :kp]), a_scale
 
@@ -244,7 +260,7 @@ def rmsnorm_quantize_i8(
         raise RuntimeError(f"{name}: weight has {weight.numel()} elements, expected {h}")
     q = torch.empty((*x.shape[:-1], kpa), dtype=torch.int8, device=dev)
     a_scale = torch.empty(x.shape[:-1], dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             "wfb_rmsnorm_quant_i8", _p(x), dt, h, _p(weight), gdt, float(eps), m, h, _p(q), kpa, kpa, _p(a_scale), _stream(dev)
         )
@@ -308,7 +324,7 @@ def bitnet_linear(
     lda = a2.stride(0) if m > 1 else k
     if kernel not in _KERNELS:
         raise ValueError(f"{name}: kernel must be one of {sorted(_KERNELS)}")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             _KERNELS[kernel], _p(packed_weights), n, k, _p(a2), m, lda, _p(a_scale), ws_dev, ws,
             _p(bias), bdt, _p(out), odt, n, _p(acc), _stream(dev),
@@ -374,7 +390,7 @@ def bitnet_linear_segmented(
         raise RuntimeError(f"{name}: bias has {bias.numel()} elements, expected {n}")
     seg = (ctypes.c_int64 * len(rows))(*rows)
     lda = a2.stride(0) if m > 1 else k
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             "wfb_linear_i2s_segmented", _p(packed_weights), n, k, len(rows), ctypes.cast(seg, ctypes.c_void_p),
             _p(scales), _p(a2), m, lda, _p(a_scale), _p(bias), bdt, _p(out), odt, n, _p(acc), _stream(dev),
@@ -421,7 +437,7 @@ def glu_rmsnorm_quantize_i8(
     _, kp, kpa, _ = _rows(name, gate, k_pad)
     q = torch.empty((*gate.shape[:-1], kpa), dtype=torch.int8, device=dev)
     a_scale = torch.empty(gate.shape[:-1], dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             "wfb_glu_rmsnorm_quant_i8", _p(g2), _p(u2), dt, ldx, _ACTS[act], _p(weight), gdt, float(eps), m, h,
             _p(q), kpa, kpa, _p(a_scale), _stream(dev),
@@ -463,7 +479,7 @@ def bitnet_linear_residual(
     lda = a2.stride(0) if m > 1 else k
     ldr = residual.stride(0) if m > 1 else n
     ldo = out.stride(0) if m > 1 else n
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_linear_i2s_residual", _p(packed_weights), n, k, _p(a2), m, lda, _p(a_scale), ws_dev, ws,
                   _p(residual), _DT[residual.dtype], ldr, _p(out), _DT[out.dtype], ldo, _stream(dev))
     return out
@@ -537,7 +553,7 @@ def rmsnorm_linear(
     elif out.dtype != out_dtype or out.shape != (m, n) or out.stride(-1) != 1:
         raise RuntimeError(f"{name}: out must be {out_dtype} [{m}, {n}] with contiguous rows")
     seg = (ctypes.c_int64 * len(rows))(*rows)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_rmsnorm_linear_i2s", _p(x), _DT[x.dtype], x.stride(0), _p(weight),
                   _DT[weight.dtype] if weight is not None else WFB_F32, float(eps), m, h, _p(packed_weights), n, k,
                   len(rows), ctypes.cast(seg, ctypes.c_void_p), _p(scales), _p(residual),
@@ -587,7 +603,7 @@ def rmsnorm_linear_glu(
         out = torch.empty((m, half), dtype=torch.float32, device=dev)
     elif out.dtype != torch.float32 or out.shape != (m, half) or out.stride(-1) != 1:
         raise RuntimeError(f"{name}: out must be float32 [{m}, {half}] with contiguous rows")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_rmsnorm_linear_i2s_glu", _p(x), _DT[x.dtype], x.stride(0), _p(weight),
                   _DT[weight.dtype] if weight is not None else WFB_F32, float(eps), m, h, _p(packed_weights), n, k,
                   _p(scales), _ACTS[act], _DT[mid_dtype], _p(out), out.stride(0), _stream(dev))
@@ -635,7 +651,7 @@ def bitnet_linear_glu(
     elif out.dtype != torch.float32 or out.shape != (m, half) or out.stride(-1) != 1:
         raise RuntimeError(f"{name}: out must be float32 [{m}, {half}] with contiguous rows")
     lda = a2.stride(0) if m > 1 else k
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_linear_i2s_glu", _p(packed_weights), n, k, _p(a2), m, lda, _p(a_scale), _p(scales),
                   _ACTS[act], _DT[mid_dtype], _p(out), out.stride(0) if m > 1 else half, _stream(dev))
     return out
@@ -681,7 +697,7 @@ def linear_grad_x(packed_weights: torch.Tensor, scale: torch.Tensor, grad: torch
     m, dt = grad.shape[0], _float_dtype(name, grad)
     out = torch.empty((m, in_features), dtype=out_dtype, device=dev)
     work = _grad_workspace(m, n, in_features, dt, 0, dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_linear_grad_x", _p(grad), dt, n, m, n, _p(packed_weights), in_features, kb * 4, _p(scale),
                   _p(out), _DT[out_dtype], in_features, _p(work), _stream(dev))
     return out
@@ -707,7 +723,7 @@ def linear_grad_w(codes: torch.Tensor, a_scale: torch.Tensor, grad: torch.Tensor
     bias = None if bias_dtype is None else torch.empty(n, dtype=bias_dtype, device=dev)
     work = _grad_workspace(m, n, in_features, dt, 1, dev)
     lda = codes.stride(0) if m > 1 else codes.shape[1]
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_linear_grad_w", _p(grad), dt, n, m, n, _p(codes), lda, _p(a_scale), in_features, _p(out),
                   _DT[out_dtype], in_features, _p(bias), _DT[bias_dtype] if bias is not None else 0, _p(work),
                   _stream(dev))
@@ -726,7 +742,7 @@ def rmsnorm_grad(x: torch.Tensor, weight: torch.Tensor, grad: torch.Tensor, eps:
     gx = torch.empty_like(x) if need_x else None
     gw = torch.empty_like(weight) if need_weight else None
     work = torch.empty(min(m, 512) * h, dtype=torch.float32, device=dev) if need_weight else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_rmsnorm_grad", _p(x), _float_dtype(name, x), _p(weight), _float_dtype(name, weight), _p(grad),
                   float(eps), m, h, _p(gx), _p(gw), _DT[weight.dtype], _p(work), _stream(dev))
     return gx, gw
@@ -778,7 +794,7 @@ def bitnet_linear_argmax(
     tokens = torch.empty(m, dtype=torch.int64, device=dev)
     wsp = _argmax_ws(name, workspace, m, n, dev)
     lda = a2.stride(0) if m > 1 else k
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_linear_i2s_argmax", _p(packed_weights), n, k, _p(a2), m, lda, _p(a_scale), ws_dev, ws,
                   _p(logits), _DT[logits_dtype], n, _p(wsp), _p(tokens), _stream(dev))
     return (tokens, logits) if return_logits else tokens
@@ -809,7 +825,7 @@ def lm_head_argmax(
     tokens = torch.empty(m, dtype=torch.int64, device=dev)
     wsp = _argmax_ws(name, workspace, m, n, dev)
     ldx = x.stride(0) if m > 1 else h
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("wfb_lm_head_argmax", _p(x), _DT[x.dtype], ldx, _p(norm_weight), gdt, float(eps), _p(weight),
                   _DT[weight.dtype], h, m, n, h, _p(logits), n, _p(wsp), _p(tokens), _stream(dev))
     return (tokens, logits) if return_logits else tokens
@@ -890,7 +906,7 @@ def gqa_decode_attention(
     ldo = out.stride(0) if b > 1 else hq * d
     sc = 1.0 / float(d) ** 0.5 if scale is None else float(scale)
     work = torch.empty(b * hq * (d + 2) * ((max_len + 63) // 64), dtype=torch.float32, device=dev) if split else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             "wfb_gqa_decode_attention", _p(q2), ldq, _p(k2), ldk, _p(v2), ldv, _DT[q.dtype], _p(rope_cos),
             _p(rope_sin), _p(k_cache), _p(v_cache), max_len, _p(pos), b, hq, hkv, d, sc, _p(out), ldo, _p(work),
@@ -948,7 +964,7 @@ def gqa_prefill_attention(
         raise RuntimeError(f"{name}: out must be [{rows}, {hq * d}] {q.dtype} with contiguous rows")
     ldo = out.stride(0) if rows > 1 else hq * d
     sc = 1.0 / float(d) ** 0.5 if scale is None else float(scale)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call(
             "wfb_gqa_prefill_attention", _p(q2), ldq, _p(k2), ldk, _p(v2), ldv, _DT[q.dtype], _p(rope_cos),
             _p(rope_sin), _p(k_cache), _p(v_cache), max_len, int(start), b, int(t), hq, hkv, d, sc, _p(out), ldo,
