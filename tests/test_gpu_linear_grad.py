@@ -38,6 +38,19 @@ def test_linear_grads_match_float64(pkg, dev, m, n, k, dtype):
         assert torch.equal(ops.linear_grad_w(codes, a_scale, gy, k, out), gw.to(out))
 
 
+@pytest.mark.parametrize("m", [520, 1030])
+def test_grad_w_splits_only_the_last_tiles(pkg, dev, m):
+    """605 tiles: 512 summed by one workgroup each and the last 93 in 2 or 5 parts, at ragged edges of both."""
+    ops, n, k = pkg.ops, 6950, 2570
+    g = torch.Generator(device=dev).manual_seed(m)
+    codes, a_scale = ops.quantize_activations_i8_per_token(torch.randn((m, k), generator=g, device=dev), k_pad=2688)
+    gy = torch.randn((m, n), generator=g, device=dev).to(torch.bfloat16)
+    gw, gb = ops.linear_grad_w(codes, a_scale, gy, k, torch.float32, torch.float32)
+    want = (gy.double() * a_scale.double()[:, None]).t().contiguous() @ codes[:, :k].double()
+    assert float((gw - want).abs().max()) <= 1e-5 * float(want.abs().max()) and _rel(gw, want) <= 1e-6
+    assert _rel(gb, gy.double().sum(0)) <= 1e-6
+
+
 def test_non_finite_gradients_reach_the_products(pkg, dev):
     """An infinite or NaN gradient gives what an fp32 product gives: inf * code, NaN where a code is 0."""
     ops = pkg.ops

@@ -13,11 +13,13 @@
 //
 // Bound by the matrix cores: one pass over grad_x and three over grad_w instead of fp32 products, which run at a
 // sixteenth of the bf16 rate.  2048 tokens, 2560 -> 6912, bf16 (traced): grad_x 549 -> 88 us + 12 for its three
-// partial sums, grad_w 549 -> 200 + 26 us, the layout kernels 40 us in place of 160 us of conversions and transposes;
-// forward and backward 1346 -> 442 us.
+// partial sums, grad_w 549 -> 189 + 6 us, the layout kernels 40 us in place of 160 us of conversions and transposes;
+// forward and backward 1396 -> 412 us.
 //
 // Two steps.  Layout kernels write the operands with the summed index contiguous (the ternary codes and the int8
 // codes transposed to bf16; g * a_scale transposed and split), zero-padded to whole stages; then the tile kernel.
+
+#include <algorithm>
 
 #include "wfb_common.h"
 
@@ -202,9 +204,11 @@ struct GradGemm {
   int I, J;
   int c_a;             // elements of an A row (offsets past it read zeros)
   int stages;          // of BK elements, all splits together
-  int nsplit;          // K splits: split s takes stages [s * per, ...), per = ceil(stages / nsplit)
+  int full;            // the first `full` tiles are summed by one workgroup each,
+  int nsplit;          // the others by nsplit: split s takes stages [s * per, ...), per = ceil(stages / nsplit)
   const float* alpha;  // device scalar or null (1)
-  void* out;           // nsplit = 1: [I][ldo] in out_dtype; else fp32 partials [nsplit][I][ldo]
+  float* parts;        // fp32 partial tiles [tiles past full][nsplit][BI][BJ]
+  void* out;           // [I][ldo] in out_dtype
   int out_dtype;
   int64_t ldo;
   bool vec;            // rows of out 16-byte aligned
@@ -245,7 +249,7 @@ __device__ __forceinline__ void store8(const GradGemm& p, int64_t off, int col, 
 // rows at one chunk meet 16 distinct bank groups), the next stage's loads in flight while a stage is multiplied.
 template <int P, int TI, int TJ, int WI, int WJ, int BK, int WPE>
 __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void grad_tile_kernel(
-    GradGemm p, int tiles_i, int tiles_j, int ntiles) {
+    GradGemm p, int tiles_i, int tiles_j) {
   constexpr int W = WI * WJ, BI = 32 * TI * WI, BJ = 32 * TJ * WJ;
   constexpr int ROW = 2 * BK, CH = ROW / 16, RPI = 64 / CH;  // bytes and chunks of a row, rows per load
   constexpr int ASZ = P * BI * ROW, BSZ = BJ * ROW, SZ = ASZ + BSZ;
@@ -258,15 +262,17 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
   const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wi = w / WJ, wj = w % WJ, i = l & 31, g = l >> 5;
 
-  const int per8 = gridDim.x / 8;  // the grid is a multiple of 8; each XCD takes a contiguous range
-  const int t = (blockIdx.x % 8) * per8 + blockIdx.x / 8;
-  if (t >= ntiles * p.nsplit) return;
-  const int split = t / ntiles, tt = t % ntiles;
+  // whole tiles first, each XCD a contiguous range of them; then the split ones
+  const int per8 = (p.full + 7) / 8, bid = blockIdx.x, u = bid - 8 * per8;
+  const bool whole = u < 0;
+  const int tt = whole ? (bid % 8) * per8 + bid / 8 : p.full + u / p.nsplit;
+  if (whole && tt >= p.full) return;
+  const int split = whole ? 0 : u % p.nsplit;
   constexpr int kGroup = 8;
   const int gsz = kGroup * tiles_j, grp = tt / gsz, rr = tt - grp * gsz;
   const int gm = min(kGroup, tiles_i - grp * kGroup);
   const int i0 = (grp * kGroup + rr % gm) * BI, j0 = (rr / gm) * BJ;
-  const int per = (p.stages + p.nsplit - 1) / p.nsplit;
+  const int per = whole ? p.stages : (p.stages + p.nsplit - 1) / p.nsplit;
   const int s0 = split * per, s1 = min(s0 + per, p.stages);
 
   const int irows = min(BI, p.I - i0), jrows = min(BJ, p.J - j0);
@@ -380,9 +386,9 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
   constexpr int WPB = SZ / ST;                     // waves whose staging fits one buffer
   static_assert(TJ % TS == 0 && WPB >= 1 && 2 * WPB >= W, "staging fits the two operand buffers");
   uint8_t* st = w < WPB ? lds0 + w * ST : lds1 + (w - WPB) * ST;
-  const float alpha = p.alpha ? p.alpha[0] : 1.0f;
+  const float alpha = whole && p.alpha ? p.alpha[0] : 1.0f;
   constexpr int LPR = CPR / 2, RP = 64 / LPR;
-  const int64_t obase = p.nsplit > 1 ? (int64_t)split * p.I * p.ldo : 0;
+  float* const part = whole ? nullptr : p.parts + (int64_t)u * (BI * BJ);
 #pragma unroll
   for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
@@ -401,29 +407,35 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
         const int r = RP * jj + l / LPR, c8 = l % LPR;
         const float4 ya = *reinterpret_cast<const float4*>(st + (r * CPR + ((2 * c8) ^ (r & (CPR - 1)))) * 16);
         const float4 yb = *reinterpret_cast<const float4*>(st + (r * CPR + ((2 * c8 + 1) ^ (r & (CPR - 1)))) * 16);
-        const int row = i0 + wi * 32 * TI + ti * 32 + r, col = j0 + (wj * TJ + ts) * 32 + 8 * c8;
-        if (row < p.I && col < p.J) store8(p, obase + (int64_t)row * p.ldo + col, col, ya, yb);
+        const int row = wi * 32 * TI + ti * 32 + r, col = (wj * TJ + ts) * 32 + 8 * c8;  // within the tile
+        if (!whole) {
+          float4* o = reinterpret_cast<float4*>(part + row * BJ + col);
+          o[0] = ya;
+          o[1] = yb;
+        } else if (i0 + row < p.I && j0 + col < p.J) {
+          store8(p, (int64_t)(i0 + row) * p.ldo + j0 + col, j0 + col, ya, yb);
+        }
       }
     }
 }
 
-// out[i][j] = alpha * sum over the splits, in order, of part[s][i][j] (rows of ldp elements, a multiple of 8)
-__global__ __launch_bounds__(256) void grad_reduce_kernel(const float* __restrict__ part, int nsplit, int64_t ldp,
-                                                          GradGemm p) {
-  const int64_t per = ldp / 8, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)p.I * per) return;
-  const int64_t row = idx / per, col = 8 * (idx % per);
-  const float* src = part + row * ldp + col;
-  const int64_t plane = (int64_t)p.I * ldp;
+// The tiles past p.full: out = alpha * the sum of a tile's parts, in order.  A workgroup sums 2048 outputs.
+__global__ __launch_bounds__(256) void grad_reduce_kernel(GradGemm p, int bi, int bj, int tiles_i, int tiles_j) {
+  const int per = bi * bj / 2048, tile = blockIdx.x / per, e = 2048 * (blockIdx.x % per) + 8 * threadIdx.x;
+  const int tt = p.full + tile, gsz = 8 * tiles_j, grp = tt / gsz, rr = tt - grp * gsz;  // the tile kernel's order
+  const int gm = min(8, tiles_i - grp * 8);
+  const int row = (grp * 8 + rr % gm) * bi + e / bj, col = (rr / gm) * bj + e % bj;
+  if (row >= p.I || col >= p.J) return;
+  const float* src = p.parts + (int64_t)tile * p.nsplit * (bi * bj) + e;
   float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-  for (int s = 1; s < nsplit; ++s) {
-    const float4 c = *reinterpret_cast<const float4*>(src + s * plane);
-    const float4 d = *reinterpret_cast<const float4*>(src + s * plane + 4);
+  for (int s = 1; s < p.nsplit; ++s) {
+    src += bi * bj;
+    const float4 c = *reinterpret_cast<const float4*>(src), d = *reinterpret_cast<const float4*>(src + 4);
     a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
     b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
   }
   const float alpha = p.alpha ? p.alpha[0] : 1.0f;
-  store8(p, row * p.ldo + col, (int)col, make_float4(a.x * alpha, a.y * alpha, a.z * alpha, a.w * alpha),
+  store8(p, (int64_t)row * p.ldo + col, col, make_float4(a.x * alpha, a.y * alpha, a.z * alpha, a.w * alpha),
          make_float4(b.x * alpha, b.y * alpha, b.z * alpha, b.w * alpha));
 }
 
@@ -440,79 +452,89 @@ struct Variant {
 };
 constexpr Variant kVariants[] = {{1, 256, 256, 64, 1, 1.20, 8}, {1, 128, 128, 64, 2, 1.05, 5},
                                  {1, 64, 128, 64, 3, 0.80, 3}, {3, 128, 256, 32, 2, 1.15, 8},
-                                 {3, 64, 128, 32, 4, 0.92, 2.5}};
+                                 {3, 64, 128, 32, 4, 0.85, 2.5}};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
+// The first `full` tiles whole, the others in nsplit parts of the summed index, each a workgroup of its own.
 struct Plan {
-  int variant, nsplit;  // nsplit: parts the summed index is cut into, each a workgroup of its own per tile
+  int variant;
+  int64_t tiles, full;
+  int nsplit;
 };
 
-// The variant and split with the least estimated time: rounds of workgroups (a last round that leaves CUs with
-// one workgroup runs it in less than the time of a full one) and, for a split, the partial sums written and read
-// back.  Swept on MI355X over every (variant, split) of 18 shapes from 1 x 576 x 576 to 4096^3, both products: the
-// estimate's pick is within 8% of the fastest on all but four, within 15% there.
+// The least estimated time of every variant, of its tiles all split (or none) or only those past the last full round
+// of workgroups, and of the number of parts: rounds of workgroups (a last round that leaves CUs with one workgroup
+// runs it in less than the time of a full one) and the partial sums written and read back.  Swept on MI355X over
+// every (variant, split of all tiles) of 18 shapes from 1 x 576 x 576 to 4096^3, both products: the estimate's pick
+// is within 8% of the fastest on all but four, within 15% there.  Splitting only the tiles past the last full round
+// (28 of 540 at 2048 x 6912 x 2560) took grad_w there from 200 us and 26 for all tiles' sums to 189 and 6.
 Plan plan(int planes, int64_t I, int64_t J, int64_t C) {
-  Plan best{-1, 1};
+  Plan best{-1, 0, 0, 1};
   double best_us = 0;
   for (int v = 0; v < kNumVariants; ++v) {
     const Variant& t = kVariants[v];
     if (t.planes != planes) continue;
     const int64_t tiles = ((I + t.bi - 1) / t.bi) * ((J + t.bj - 1) / t.bj), slots = 256 * t.per_cu;
     const int64_t stages = pad_to(C, kPad) / t.bk;
-    for (int64_t want = 1; want <= 16 && (want == 1 || stages / want >= 4); ++want) {
-      const int64_t per = (stages + want - 1) / want, ns = (stages + per - 1) / per;  // no empty split
-      if (ns != want) continue;
-      const int64_t wgs = tiles * ns, full = wgs / slots;
+    const double rate = t.rate * 1e9 / slots;  // operations per us of one workgroup's slot
+    auto rounds_us = [&](int64_t wgs, int64_t n) {  // wgs workgroups of n stages each
+      const int64_t full = wgs / slots;
       const double r = (double)(wgs % slots) / slots;
       const double last = r == 0 ? 0 : t.per_cu == 1 ? 0.85 : r * t.per_cu <= 1 ? 0.6 : 0.6 + 0.4 * r;
-      const double flop = 2.0 * planes * t.bi * t.bj * per * t.bk * slots;
-      double us = (full + last) * flop / (t.rate * 1e9) + t.round_us * (full + (r > 0));
-      if (ns > 1) us += 4.0 + 8.0 * ns * I * J / 8e6;
-      if (best.variant < 0 || us < best_us) best = {v, (int)ns}, best_us = us;
+      return (full + last) * 2.0 * planes * t.bi * t.bj * n * t.bk / rate + t.round_us * (full + (r > 0));
+    };
+    auto consider = [&](int64_t full, int64_t ns, double us) {
+      if (best.variant < 0 || us < best_us) best = {v, tiles, full, (int)ns}, best_us = us;
+    };
+    consider(tiles, 1, rounds_us(tiles, stages));
+    for (int64_t want = 2; want <= 32 && stages / want >= 4; ++want) {
+      const int64_t per = (stages + want - 1) / want, ns = (stages + per - 1) / per;  // no empty split
+      if (ns != want) continue;
+      for (const int64_t full : {(int64_t)0, tiles / slots * slots}) {
+        const int64_t rest = tiles - full;
+        if (rest == 0 || rest * ns > 4 * slots) continue;  // (no rest, or enough workgroups without so many parts)
+        const double sums = 4.0 + 8.0 * ns * rest * t.bi * t.bj / 8e6;
+        consider(full, ns, (full ? rounds_us(full, stages) : 0) + rounds_us(rest * ns, per) + sums);
+      }
     }
   }
   return best;
 }
 
 template <int P, int TI, int TJ, int WI, int WJ, int BK, int WPE>
-hipError_t launch_tiles(const GradGemm& p, hipStream_t s) {
-  const int ti = (p.I + 32 * TI * WI - 1) / (32 * TI * WI), tj = (p.J + 32 * TJ * WJ - 1) / (32 * TJ * WJ);
-  const int64_t n = (int64_t)ti * tj, grid = pad_to(n * p.nsplit, 8);
+hipError_t launch_tiles(const GradGemm& p, const Plan& pl, hipStream_t s) {
+  constexpr int BI = 32 * TI * WI, BJ = 32 * TJ * WJ;
+  const int ti = (p.I + BI - 1) / BI, tj = (p.J + BJ - 1) / BJ;
+  const int64_t rest = pl.tiles - pl.full, grid = pad_to(pl.full, 8) + rest * pl.nsplit;
   if (grid > INT32_MAX) return hipErrorInvalidValue;
   hipLaunchKernelGGL((grad_tile_kernel<P, TI, TJ, WI, WJ, BK, WPE>), dim3((unsigned)grid), dim3(64 * WI * WJ), 0, s, p,
-                     ti, tj, (int)n);
+                     ti, tj);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || rest == 0) return e;
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)(rest * (BI * BJ / 2048))), dim3(256), 0, s, p, BI, BJ, ti, tj);
   return hipGetLastError();
 }
 
 hipError_t run_gemm(GradGemm p, const Plan& pl, int64_t C, float* parts, hipStream_t s) {
   p.stages = (int)(pad_to(C, kPad) / kVariants[pl.variant].bk);
+  p.full = (int)pl.full;
   p.nsplit = pl.nsplit;
+  p.parts = parts;
   const int osz = p.out_dtype == WFB_F32 ? 4 : 2;
   p.vec = (uintptr_t)p.out % 16 == 0 && (p.ldo * osz) % 16 == 0;
-  GradGemm q = p;
-  if (pl.nsplit > 1) {
-    q.alpha = nullptr;
-    q.out = parts;
-    q.out_dtype = WFB_F32;
-    q.ldo = pad_to(p.J, 8);
-    q.vec = true;
-  }
-  hipError_t e;
   switch (pl.variant) {  // kVariants
-    case 0: e = launch_tiles<1, 4, 2, 2, 4, 64, 2>(q, s); break;
-    case 1: e = launch_tiles<1, 2, 2, 2, 2, 64, 2>(q, s); break;
-    case 2: e = launch_tiles<1, 1, 2, 2, 2, 64, 3>(q, s); break;
-    case 3: e = launch_tiles<3, 2, 4, 2, 2, 32, 2>(q, s); break;
-    default: e = launch_tiles<3, 1, 2, 2, 2, 32, 4>(q, s); break;
+    case 0: return launch_tiles<1, 4, 2, 2, 4, 64, 2>(p, pl, s);
+    case 1: return launch_tiles<1, 2, 2, 2, 2, 64, 2>(p, pl, s);
+    case 2: return launch_tiles<1, 1, 2, 2, 2, 64, 3>(p, pl, s);
+    case 3: return launch_tiles<3, 2, 4, 2, 2, 32, 2>(p, pl, s);
+    default: return launch_tiles<3, 1, 2, 2, 2, 32, 4>(p, pl, s);
   }
-  if (e != hipSuccess || pl.nsplit == 1) return e;
-  const int64_t items = (int64_t)p.I * (q.ldo / 8);
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, parts, pl.nsplit, q.ldo, p);
-  return hipGetLastError();
 }
 
 constexpr int64_t align256(int64_t b) { return pad_to(b, 256); }
-int64_t part_bytes(const Plan& pl, int64_t I, int64_t J) { return pl.nsplit > 1 ? 4 * pl.nsplit * I * pad_to(J, 8) : 0; }
+int64_t part_bytes(const Plan& pl) {
+  return 4 * (pl.tiles - pl.full) * pl.nsplit * kVariants[pl.variant].bi * kVariants[pl.variant].bj;
+}
 
 int grad_x_planes(int gdt) { return gdt == WFB_BF16 ? 1 : 3; }
 
@@ -523,13 +545,13 @@ int grad_x_planes(int gdt) { return gdt == WFB_BF16 ? 1 : 3; }
 int64_t grad_x_workspace(int64_t m, int64_t n, int64_t k, int gdt) {
   const int64_t np = pad_to(n, kPad);
   const int P = grad_x_planes(gdt);
-  return align256(2 * k * np) + align256(2 * P * m * np) + part_bytes(plan(P, m, k, n), m, k);
+  return align256(2 * k * np) + align256(2 * P * m * np) + part_bytes(plan(P, m, k, n));
 }
 
 int64_t grad_w_workspace(int64_t m, int64_t n, int64_t k) {
   const int64_t mp = pad_to(m, kPad);
   return align256(2 * 3 * n * mp) + align256(2 * k * mp) + align256(4 * (mp / 64) * n) +
-         part_bytes(plan(3, n, k, m), n, k);
+         part_bytes(plan(3, n, k, m));
 }
 
 hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const uint8_t* qw, int64_t k,
