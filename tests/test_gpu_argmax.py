@@ -66,6 +66,23 @@ def test_persistent_head_accumulators(pkg, dev, m, n, k):
     assert np.array_equal(y.cpu().numpy(), orc.rescale(acc_ref, np.float32(ws), a_scale))
 
 
+# plain outputs of 32768 rows and more: persistent from 8 tokens of 2560 (5 waves; 2528 pads to 2560, 3712: 8 waves, the
+# last short), one-shot below, at the edges of the rule and with a ragged last row tile
+@pytest.mark.parametrize("m,n,k", [(7, 32768, 2560), (8, 32768, 2560), (8, 32799, 2528), (16, 33009, 3712), (9, 65537, 4096),
+                                   (16, 32767, 4096), (17, 32768, 2560)])
+@pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
+def test_plain_head_outputs_match_oracle(pkg, dev, m, n, k, odt):
+    rng = np.random.default_rng(m + n + k)
+    k_pad = -(-k // 128) * 128
+    w, a = orc.random_ternary(rng, n, k_pad), np.zeros((m, k_pad), np.int8)
+    w[:, k:], a[:, :k] = 0, orc.random_int8(rng, m, k)
+    packed, ws, a_scale = orc.pack_i2s(w), orc.log_uniform(rng), orc.log_uniform(rng, m)
+    acc = (a.astype(np.float32) @ w.astype(np.float32).T).astype(np.int64)  # exact: partial sums below 2^24
+    y = pkg.bitnet_linear(torch.from_numpy(packed).to(dev), torch.from_numpy(a).to(dev), float(ws),
+                          a_scale=torch.from_numpy(a_scale).to(dev), out_dtype=odt)
+    assert torch.equal(y.cpu(), torch.from_numpy(orc.rescale(acc, np.float32(ws), a_scale)).to(odt))
+
+
 def test_ternary_head_argmax_ties_pick_first(pkg, dev):
     rng = np.random.default_rng(3)
     n, k = 777, 512

@@ -1005,9 +1005,14 @@ hipError_t launch_modes(const uint8_t* W, int n, int C, const int8_t* A, int m, 
                         int nt_pref, const NormSrc& ns, hipStream_t s) {
   if (ns.x == nullptr) {
     if (A == nullptr) return hipErrorInvalidValue;
-    // many row tiles with a per-lane epilogue (the greedy LM head): the persistent form (one token tile)
+    // many row tiles (the LM head): the persistent form (one token tile), always with a per-lane epilogue (greedy keys,
+    // accumulators), for plain outputs where the one-shot form's activation staging costs more than its whole-line
+    // stores save: from 8 tokens of 2560 or more (cold weights on MI355X, one-shot against persistent: 128256 x 4096
+    // at M = 8 36.3 -> 27.2 us, M = 16 45.0 -> 29.5; x 2560 28.6 -> 26.3 and 30.2 -> 26.9, but M = 4 21.6 -> 25.7;
+    // 32768 x 2048 at M = 16 6.8 -> 9.3, 49152 x 640 7.0 -> 12.1)
     if constexpr (MR <= 16) {
-      if (GLUE == 0 && (e.amax || e.acc_out || !e.out) && !e.bias && !e.res && e.nseg == 1 && n >= kPersistMinRows) {
+      const bool lanes = e.amax || e.acc_out || !e.out;
+      if (GLUE == 0 && (lanes || (m >= 8 && C >= 40)) && !e.bias && !e.res && e.nseg == 1 && n >= kPersistMinRows) {
         const hipError_t st = launch_persist(W, n, C, A, m, lda, e, cu_count(), s);
         if (st != hipErrorNotSupported) return st;
       }

@@ -501,10 +501,13 @@ def rmsnorm_linear_glu_supported(m: int, h: int, k: int) -> bool:
 
 
 def rmsnorm_linear_preferred(m: int, h: int, n: int, k: int, gamma_bytes: int = 2) -> bool:
-    """Whether the fused launch is the faster choice: every supported size (measured on MI355X, the prologue
-    costs less than the separate quantiser launch it replaces at the Llama-3-8B, BitNet-2B and SmolLM2
-    decode shapes)."""
-    return rmsnorm_linear_supported(m, h, k, gamma_bytes)
+    """Whether the fused launch is the faster choice.  Its workgroups each repeat the norm, which up to some 32768
+    output rows costs less than the separate quantiser launch it replaces (measured on MI355X at the Llama-3-8B,
+    BitNet-2B and SmolLM2 decode shapes) and on a vocabulary's rows more: quantiser and linear against fused, cold
+    weights, 128256 x 4096 at M = 1 / 8 / 16 25 / 33 / 35 us against 30 / 50 / 86, 49152 x 640 at M = 3 / 16 7.3 / 9.7
+    against 12.8 / 35; 32768 x 2048 at M = 2 / 4 10.9 / 9.7 against 8.4 / 8.5, M = 8 9.8 against 10.3."""
+    wide = n >= 65536 or (n >= 32768 and m * n >= 147456)
+    return not wide and rmsnorm_linear_supported(m, h, k, gamma_bytes)
 
 
 def rmsnorm_linear(
