@@ -102,6 +102,24 @@ def test_pack_given_scale_and_ties(pkg, dev):
     assert np.array_equal(qw.cpu().numpy(), orc.pack_i2s(orc.ternarize(w, 1.0)))
 
 
+# rows of fewer, exactly and more than 256 packed dwords (workgroup edges), a last workgroup that is not full
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k", [(1, 128), (67, 128), (13, 2560), (5, 4096), (7, 4224), (3, 12288)])
+def test_pack_codes_around_half_a_scale(pkg, dev, dtype, n, k):
+    """Weights at, next to and on either side of half a scale, scales of every kind: the oracle's quotients (exact)."""
+    rng = np.random.default_rng(n + k)
+    for s in (np.float32(0.731), np.float32(2.0**-126), np.float32(3e-42), np.float32(2e38), np.float32(-0.25), np.float32(np.inf)):
+        h = np.float32(s * np.float32(0.5))
+        with np.errstate(all="ignore"):
+            near = np.array([h, np.nextafter(h, np.float32(0)), np.nextafter(h, np.float32(np.inf)), s, h / 2, 0, 1.0, 3e38], np.float32)
+            near = near[np.isfinite(near)]
+            w = torch.from_numpy(rng.choice(near, (n, k)) * rng.choice(np.array([-1, 1], np.float32), (n, k))).to(dtype)
+            w[w.isinf()] = 1.0  # (16-bit roundings of the largest floats: over an infinite scale they have no quotient)
+            ref = orc.pack_i2s(orc.ternarize(w.float().numpy(), s))
+        qw, _ = pkg.pack_ternary_i2s(w.to(dev), scale=torch.full((1,), float(s), device=dev))
+        assert np.array_equal(qw.cpu().numpy(), ref), s
+
+
 def test_absmean_tiny_weights(pkg, dev):
     w = torch.full((8, 128), 1e-9, device=dev)
     assert pkg.absmean_scale(w).item() == 1.0

@@ -71,35 +71,55 @@ __global__ __launch_bounds__(256) void absmean_final_kernel(const double* __rest
   }
 }
 
+// clamp(rint(w / s), -1, 1) + 1 of the correctly rounded quotient; NaN gives 0.
 __device__ __forceinline__ uint32_t ternary_code(float w, float s) {
   float q = __builtin_rintf(__fdiv_rn(w, s));
   q = fminf(fmaxf(q, -1.0f), 1.0f);
   return (uint32_t)((int)q + 1);
 }
 
-// One thread per output dword: bytes j..j+3 (j = 4*(p % 8)) of block b = p / 8 of row `row`.
+// The same code for h = s / 2 of a finite s >= 2^-125 (h is exact then): rint gives 1 where the quotient rounds to more
+// than 1/2, which is where w / s > 1/2 + 2^-25 (a tie goes to the even 1/2), that is w > h + h 2^-24 -- a bound within
+// [h + ulp(h) / 2, h + ulp(h)), which the floats above h, and only they, exceed.  NaN fails both comparisons.
+__device__ __forceinline__ uint32_t ternary_code_half(float w, float h) { return w > h ? 2u : w >= -h ? 1u : 0u; }
+
+// One thread per output dword: bytes j..j+3 (j = 4*(p % 8)) of block b = p / 8 of row `row`.  A pass over the weights:
+// with a division per weight and 64-bit index divisions per thread, 16-bit weights were bound by those (6912 x 2560
+// bf16 13.0 us); with the comparisons and one uniform 64-bit division per workgroup 8.9.  fp32 weights are bound by the
+// reads before and after (14336 x 4096 36.5 us, 6.4 TB/s).
 template <int DT>
 __global__ __launch_bounds__(256) void pack_i2s_kernel(const void* __restrict__ w, int64_t n, int64_t k,
                                                        int64_t ldw, const float* __restrict__ scale,
                                                        uint32_t* __restrict__ qw) {
   const int64_t dw_per_row = k / 16;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= n * dw_per_row) return;
-  const int64_t row = gid / dw_per_row;
-  const int64_t p = gid % dw_per_row;
+  const int64_t first = (int64_t)blockIdx.x * 256, row0 = first / dw_per_row;
+  int64_t row = row0, p = first - row0 * dw_per_row + threadIdx.x;
+  if (dw_per_row < 256) {  // rows end within the workgroup, more than once for the shortest
+    row += (uint32_t)p / (uint32_t)dw_per_row;
+    p = (uint32_t)p % (uint32_t)dw_per_row;
+  } else if (p >= dw_per_row) {
+    row += 1;
+    p -= dw_per_row;
+  }
+  if (row >= n) return;
   const int64_t b = p >> 3;
   const int j = (int)(p & 7) * 4;
   const float s = scale[0];
+  const bool plain = s >= 0x1p-125f && s <= 0x1.fffffep127f;
+  const float h = 0.5f * s;
   const int64_t base = row * ldw + 128 * b + j;
+  float v[4][4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[f][t] = load_elem<DT>(w, base + 32 * f + t);
   uint32_t out = 0;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    uint32_t byte = 0;
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int f = 0; f < 4; ++f) byte |= ternary_code(load_elem<DT>(w, base + 32 * f + t), s) << (6 - 2 * f);
-    out |= byte << (8 * t);
-  }
-  qw[gid] = out;
+    for (int f = 0; f < 4; ++f)
+      out |= (plain ? ternary_code_half(v[f][t], h) : ternary_code(v[f][t], s)) << (8 * t + 6 - 2 * f);
+  qw[first + threadIdx.x] = out;
 }
 
 __global__ __launch_bounds__(256) void unpack_i2s_kernel(const uint8_t* __restrict__ qw, int64_t n, int64_t k,
