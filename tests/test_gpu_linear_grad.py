@@ -87,6 +87,30 @@ def test_gradients_of_gradients_and_batched_gradients_keep_working(pkg, dev):
     assert _rel(bx[0], plain[0].double()) <= 1e-6 and _rel(bw[1], 2 * plain[1].double()) <= 1e-6
 
 
+def _module(pkg, dev, subln):
+    """(module with a bias, input, the tensors to differentiate) of a small layer."""
+    torch.manual_seed(11)
+    mod = (pkg.SubLNBitLinear if subln else pkg.BitLinear)(256, 96, bias=True, device=dev)
+    lin = mod.linear if subln else mod
+    x = torch.randn(7, 256, device=dev, requires_grad=True)
+    return mod, x, [x, lin.weight, lin.bias] + ([mod.norm_weight] if subln else [])
+
+
+@pytest.mark.parametrize("subln", [False, True])
+def test_forward_mode_tangents_pass_through_the_backward(pkg, dev, subln):
+    """Every gradient is linear in the output's: its tangent is the gradient at the tangent (the two routes' fp32
+    sums differ by 1e-6 at most)."""
+    from torch.autograd import forward_ad as fw
+
+    mod, x, wrt = _module(pkg, dev, subln)
+    gy, t = torch.randn(7, 96, device=dev), torch.randn(7, 96, device=dev)
+    with fw.dual_level():
+        grads = torch.autograd.grad(mod(x), wrt, fw.make_dual(gy, t))
+        tangents = [fw.unpack_dual(g).tangent for g in grads]
+    for got, want in zip(tangents, torch.autograd.grad(mod(x), wrt, t)):
+        assert got is not None and _rel(got, want.double()) <= 1e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
 def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):

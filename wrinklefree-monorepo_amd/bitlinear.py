@@ -27,6 +27,7 @@ from typing import Callable, Iterable, List, Optional
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from .ops import (
     QK_I2_S,
@@ -72,9 +73,11 @@ def _out_dtype(x: torch.Tensor) -> torch.dtype:
 
 def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
     """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
-    backward is itself being differentiated (create_graph) or batched by a functorch transform: those take the torch
-    products, which autograd and vmap see through."""
-    return not torch.is_grad_enabled() and linear_grad_supported(gy, in_features)
+    backward is itself being differentiated (create_graph, forward mode) or batched by a functorch transform: those
+    take the torch products, which autograd and vmap see through."""
+    if torch.is_grad_enabled() or forward_ad._current_level >= 0:
+        return False
+    return linear_grad_supported(gy, in_features)
 
 
 def _weight_grads(q: torch.Tensor, a_scale: torch.Tensor, gy: torch.Tensor, kin: int, wdt: torch.dtype,
