@@ -111,6 +111,20 @@ def test_forward_mode_tangents_pass_through_the_backward(pkg, dev, subln):
         assert got is not None and _rel(got, want.double()) <= 1e-6
 
 
+@pytest.mark.parametrize("subln", [False, True])
+def test_traced_backward_computes_the_weight_gradients(pkg, dev, subln):
+    """A traced backward holds the products of its inputs: on another output gradient it gives that one's weight and
+    bias gradients (fp32 sums in another order: 1e-6)."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    mod, x, wrt = _module(pkg, dev, subln)
+    y = mod(x)
+    gy, other = torch.randn(7, 96, device=dev), torch.randn(7, 96, device=dev)
+    traced = make_fx(lambda g: torch.autograd.grad(y, wrt[1:3], g, retain_graph=True))(gy)
+    for got, want in zip(traced(other), torch.autograd.grad(y, wrt[1:3], other)):
+        assert _rel(got, want.double()) <= 1e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
 def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):

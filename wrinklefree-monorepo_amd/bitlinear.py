@@ -73,9 +73,9 @@ def _out_dtype(x: torch.Tensor) -> torch.dtype:
 
 def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
     """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
-    backward is itself being differentiated (create_graph, forward mode) or batched by a functorch transform: those
-    take the torch products, which autograd and vmap see through."""
-    if torch.is_grad_enabled() or forward_ad._current_level >= 0:
+    backward is itself being differentiated (create_graph, forward mode), batched by a functorch transform or watched
+    by a dispatch mode (a tracer): those take the torch products, which all of them see through."""
+    if torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
         return False
     return linear_grad_supported(gy, in_features)
 
