@@ -125,6 +125,36 @@ def test_traced_backward_computes_the_weight_gradients(pkg, dev, subln):
         assert _rel(got, want.double()) <= 1e-6
 
 
+class _Wrapped(torch.Tensor):
+    """A tensor subclass without memory of its own: every operation runs on the tensor inside."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, dtype=inner.dtype, device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        from torch.utils._pytree import tree_map
+
+        def unwrap(v):
+            return v.inner if isinstance(v, cls) else v
+
+        out = func(*tree_map(unwrap, args), **tree_map(unwrap, kwargs or {}))
+        return tree_map(lambda v: cls(v) if isinstance(v, torch.Tensor) else v, out)
+
+
+@pytest.mark.parametrize("subln", [False, True])
+def test_subclass_gradients_take_the_torch_products(pkg, dev, subln):
+    mod, x, wrt = _module(pkg, dev, subln)
+    gy = torch.randn(7, 96, device=dev)
+    grads = torch.autograd.grad(mod(x), wrt, _Wrapped(gy))
+    for got, want in zip(grads, torch.autograd.grad(mod(x), wrt, gy)):
+        assert _rel(got.inner, want.double()) <= 1e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
 def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):

@@ -74,8 +74,11 @@ def _out_dtype(x: torch.Tensor) -> torch.dtype:
 def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
     """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
     backward is itself being differentiated (create_graph, forward mode), batched by a functorch transform or watched
-    by a dispatch mode (a tracer): those take the torch products, which all of them see through."""
+    by a dispatch mode (a tracer), nor for a gradient of a tensor subclass (its memory, if it has any, is the class's
+    own affair): those take the torch products, which all of them see through."""
     if torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
+        return False
+    if type(gy) not in (torch.Tensor, nn.Parameter):
         return False
     return linear_grad_supported(gy, in_features)
 
