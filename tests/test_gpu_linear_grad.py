@@ -155,6 +155,29 @@ def test_subclass_gradients_take_the_torch_products(pkg, dev, subln):
         assert _rel(got.inner, want.double()) <= 1e-6
 
 
+def _negated_view(t):
+    """t's values as a lazily negated, strided view (what .imag of a conjugate is)."""
+    return torch.complex(torch.zeros_like(t), -t).conj().imag
+
+
+@pytest.mark.parametrize("subln", [False, True])
+@pytest.mark.parametrize("form", ["negated", "columns"])
+def test_saved_tensor_hooks_may_change_the_form(pkg, dev, subln, form):
+    """Hooks that give the float tensors back as negated views (the one-element weight scale among them), or the
+    activations and their codes column by column: the same values, the same gradients."""
+    def unpack(t):
+        if form == "negated":
+            return _negated_view(t) if t.dtype == torch.float32 else t
+        return t.t().contiguous().t() if t.dim() == 2 and t.dtype != torch.uint8 else t
+
+    mod, x, wrt = _module(pkg, dev, subln)
+    gy = torch.randn(7, 96, device=dev)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = mod(x)
+    for got, want in zip(torch.autograd.grad(y, wrt, gy), torch.autograd.grad(mod(x), wrt, gy)):
+        assert _rel(got, want.double()) <= 1e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
 def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):

@@ -71,14 +71,17 @@ def _out_dtype(x: torch.Tensor) -> torch.dtype:
     return torch.float32 if x.dtype == torch.float32 else torch.bfloat16
 
 
-def _kernel_grads(gy: torch.Tensor, in_features: int) -> bool:
+def _kernel_grads(gy: torch.Tensor, in_features: int, *saved: torch.Tensor) -> bool:
     """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
     backward is itself being differentiated (create_graph, forward mode), batched by a functorch transform or watched
     by a dispatch mode (a tracer), nor for a gradient of a tensor subclass (its memory, if it has any, is the class's
-    own affair): those take the torch products, which all of them see through."""
+    own affair), nor where a saved-tensor hook gives the saved tensors back in another form than theirs: those take
+    the torch products, which see through all of it."""
     if torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
         return False
     if type(gy) not in (torch.Tensor, nn.Parameter):
+        return False
+    if any(not t.is_contiguous() or t.is_neg() for t in saved):
         return False
     return linear_grad_supported(gy, in_features)
 
@@ -113,7 +116,7 @@ class _BitLinearSTE(torch.autograd.Function):
         q, a_scale, qweight, wscale = ctx.saved_tensors
         xdt, wdt, bdt, kin = ctx.meta
         gx = gw = gb = None
-        if _kernel_grads(gy, kin):
+        if _kernel_grads(gy, kin, q, a_scale, qweight, wscale):
             gy = gy.contiguous()
             if ctx.needs_input_grad[0]:
                 gx = linear_grad_x(qweight, wscale, gy, kin, xdt)
@@ -150,14 +153,14 @@ class _SubLNBitLinearSTE(torch.autograd.Function):
     def backward(ctx, gy):
         x2, gamma, q, a_scale, qweight, wscale = ctx.saved_tensors
         wdt, bdt, kin, eps = ctx.meta
-        if _kernel_grads(gy, kin):
+        if _kernel_grads(gy, kin, x2, gamma, q, a_scale, qweight, wscale):
             gy = gy.contiguous()
             gw, gb = _weight_grads(q, a_scale, gy, kin, wdt, bdt, *ctx.needs_input_grad[2:4])
             gx = gg = None
             if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
                 # gradient at the norm's output (identity through the quantiser), then the norm's own
                 g_norm = linear_grad_x(qweight, wscale, gy, kin, torch.float32)
-                gx, gg = rmsnorm_grad(x2.detach().contiguous(), gamma.detach().contiguous(), g_norm, eps, *ctx.needs_input_grad[:2])
+                gx, gg = rmsnorm_grad(x2.detach(), gamma.detach(), g_norm, eps, *ctx.needs_input_grad[:2])
             return gx, gg, gw, gb, None, None
         g = gy.to(torch.float32).contiguous()
         gx = gg = gw = gb = None
