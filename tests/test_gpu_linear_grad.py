@@ -178,6 +178,20 @@ def test_saved_tensor_hooks_may_change_the_form(pkg, dev, subln, form):
         assert _rel(got, want.double()) <= 1e-6
 
 
+@pytest.mark.parametrize("subln", [False, True])
+def test_negated_gradients_keep_their_sign(pkg, dev, subln):
+    """A lazily negated gradient, as strides let it through to the kernels: one element, whose view counts as
+    contiguous."""
+    mod = (pkg.SubLNBitLinear if subln else pkg.BitLinear)(256, 1, device=dev)
+    x = torch.randn(1, 256, device=dev, requires_grad=True)
+    wrt = [x, (mod.linear if subln else mod).weight]
+    gy = torch.randn(1, 1, device=dev)
+    view = _negated_view(gy)
+    assert view.is_neg() and view.is_contiguous() and torch.equal(view, gy)
+    for got, want in zip(torch.autograd.grad(mod(x), wrt, view), torch.autograd.grad(mod(x), wrt, gy)):
+        assert _rel(got, want.double()) <= 1e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,h", [(1, 8), (3, 2048), (7, 2056), (513, 576), (1100, 4104), (20, 8200), (5, 16384)])
 def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):

@@ -75,11 +75,11 @@ def _kernel_grads(gy: torch.Tensor, in_features: int, *saved: torch.Tensor) -> b
     """Whether a backward's products run on the gradient kernels (linear_grad_x / linear_grad_w).  Not when the
     backward is itself being differentiated (create_graph, forward mode), batched by a functorch transform or watched
     by a dispatch mode (a tracer), nor for a gradient of a tensor subclass (its memory, if it has any, is the class's
-    own affair), nor where a saved-tensor hook gives the saved tensors back in another form than theirs: those take
+    own affair) or a lazily negated one (its memory holds the other sign), nor where a saved-tensor hook gives the saved tensors back in another form than theirs: those take
     the torch products, which see through all of it."""
     if torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
         return False
-    if type(gy) not in (torch.Tensor, nn.Parameter):
+    if type(gy) not in (torch.Tensor, nn.Parameter) or gy.is_neg():
         return False
     if any(not t.is_contiguous() or t.is_neg() for t in saved):
         return False
