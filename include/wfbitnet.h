@@ -391,8 +391,8 @@ int wfb_linear_grad_w(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_
 /* Backward of y = x * r * gamma, r = (mean(x^2) + eps)^(-1/2) (WF/models/subln.py:42-59), in fp32:
  *   grad_x = r * (g * gamma) - x * r^3 * mean(g * gamma * x),  grad_gamma[h] = sum_m g * x * r.
  * x [M, H] (contiguous, H a multiple of 8 up to WFB_NORM_MAX_H), gamma [H], g fp32 [M, H] 16-byte aligned; grad_x of
- * x's type, 16-byte aligned, or NULL; grad_gamma of type ggamma_dtype or NULL.  work: with grad_gamma, 16-byte
- * aligned, min(M, 512) * H floats. */
+ * x's type, 16-byte aligned, or NULL; grad_gamma of type ggamma_dtype or NULL (zeros for M = 0).  work: with
+ * grad_gamma, 16-byte aligned, min(M, 512) * H floats. */
 int wfb_rmsnorm_grad(const void* x, int x_dtype, const void* gamma, int gamma_dtype, const float* g, float eps,
                      int64_t m, int64_t h, void* grad_x, void* grad_gamma, int ggamma_dtype, float* work,
                      void* stream);

@@ -210,3 +210,16 @@ def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):
         assert a.dtype == dtype and _rel(a, b) <= tol
     only = pkg.ops.rmsnorm_grad(x, w, gy, 1e-6, need_x=False)
     assert only[0] is None and torch.equal(only[1], got[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h", [8, 1000, 16384])
+def test_rmsnorm_grad_of_no_rows_is_zero(pkg, dev, dtype, h):
+    gw = torch.full((h,), 7.0, dtype=dtype, device=dev)
+    code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    pkg._lib.call("wfb_rmsnorm_grad", None, code, None, code, None, 1e-6, 0, h, None, gw.data_ptr(), code, None,
+                  torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(gw, torch.zeros_like(gw))
+    x, w = torch.empty((0, h), dtype=dtype, device=dev), torch.ones(h, dtype=dtype, device=dev)
+    gx, gw = pkg.ops.rmsnorm_grad(x, w, torch.empty((0, h), device=dev), 1e-6)
+    assert gx.shape == (0, h) and torch.equal(gw, torch.zeros_like(w))

@@ -263,7 +263,10 @@ int wfb_rmsnorm_grad(const void* x, int x_dtype, const void* gamma, int gamma_dt
     return fail(WFB_EINVAL, "%s: bad dtype", name);
   if (m < 0 || m > INT32_MAX / 2 || h <= 0 || h > WFB_NORM_MAX_H || h % 8 != 0)
     return fail(WFB_EINVAL, "%s: H (%lld) must be a multiple of 8 in 8..%d", name, (long long)h, WFB_NORM_MAX_H);
-  if (m == 0) return ok();
+  if (m == 0)  // no rows: grad_gamma is a sum of nothing
+    return grad_gamma ? hip_status(wfb::launch_column_sum(nullptr, 0, h, grad_gamma, ggamma_dtype, as_stream(stream)),
+                                   name)
+                      : ok();
   if (!x || !gamma || !g || (!grad_x && !grad_gamma) || (grad_gamma && !work))
     return fail(WFB_EINVAL, "%s: null pointer", name);
   if (!aligned(g, 16) || !aligned(grad_x, 16) || !aligned(work, 16))
