@@ -181,3 +181,18 @@ def test_many_workgroups_take_the_32_token_form(pkg, dev, d, g, t, start, scale)
     assert torch.equal(kc_d.cpu(), kc_ref) and torch.equal(vc_d.cpu().view(torch.int16), vc_ref.view(torch.int16))
     err = (out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-2)
     assert float(err.max()) <= 1e-2 and float(err.mean()) <= 2e-3
+
+
+def test_tiny_scales_of_huge_scores(pkg, dev):
+    """Queries and keys of 1e16 under a scale of 1e-33, the 32-token form (more than 512 keys): the scale counts as it
+    is, down to the smallest floats."""
+    t, hkv, g, d, scale = 700, 2, 2, 64, 1e-33
+    gen = torch.Generator().manual_seed(8)
+    q = (torch.randn((t, hkv * g * d), generator=gen) * 1e16).to(torch.bfloat16)
+    k_new = (torch.randn((t, hkv * d), generator=gen) * 1e16).to(torch.bfloat16)
+    v_new = torch.randn((t, hkv * d), generator=gen).to(torch.bfloat16)
+    kc, vc = (torch.zeros((1, hkv, t, d), dtype=torch.bfloat16) for _ in range(2))
+    ref, _, _ = _reference(q, k_new, v_new, kc, vc, 0, t, None, None, hkv * g, scale)
+    out = pkg.gqa_prefill_attention(q.to(dev), k_new.to(dev), v_new.to(dev), kc.to(dev), vc.to(dev), 0, t, scale=scale)
+    err = (out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-2)
+    assert float(err.max()) <= 1e-2 and float(err.mean()) <= 2e-3

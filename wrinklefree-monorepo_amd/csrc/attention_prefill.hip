@@ -167,8 +167,8 @@ __global__ __launch_bounds__(64 * G * QW) __attribute__((amdgpu_waves_per_eu(2))
   const int qpos32 = (int)qpos;                // positions < max_len < 2^23 (host-checked)
   const int qpos_first = (int)(start + iw);    // the wave's first query position
   // exp(s scale - m) as one fma and one exp2: scores in units of scale * log2(e), a negative scale moved into the
-  // signs of Q (exact); the floor keeps a masked score's -inf * c2 from being NaN at scale 0
-  const float c2 = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  // signs of Q (exact); the floor, the smallest normal float, keeps a masked score's -inf * c2 from being NaN at scale 0
+  const float c2 = fmaxf(fabsf(scale) * 1.4426950408889634f, 0x1p-126f);
   const uint32_t flip = scale < 0.0f ? 0x80008000u : 0u;
 
   // roped query fragments: lane holds Q[qi][16ks + 8grp .. +7] for each ks
