@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void codes_t_kernel(const int8_t* __restrict__
 __global__ __launch_bounds__(256) void weight_codes_t_kernel(const uint8_t* __restrict__ qw, int64_t row_bytes,
                                                              int64_t N, int64_t K, int64_t np,
                                                              uint16_t* __restrict__ dst) {
-  __shared__ uint8_t tile[64][36];
+  __shared__ __attribute__((aligned(4))) uint8_t tile[64][36];
   const int64_t n0 = (int64_t)blockIdx.x * 64, b = blockIdx.y;
   {
     const int r = threadIdx.x >> 2, c8 = threadIdx.x & 3;  // 8 bytes of one row per thread
