@@ -389,6 +389,11 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
   const float alpha = whole && p.alpha ? p.alpha[0] : 1.0f;
   constexpr int LPR = CPR / 2, RP = 64 / LPR;
   float* const part = whole ? nullptr : p.parts + (int64_t)u * (BI * BJ);
+  auto wave_sync = [] {  // orders the wave's LDS accesses for the compiler (the LDS keeps a wave's order by itself)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
 #pragma unroll
   for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
@@ -402,6 +407,7 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
           *reinterpret_cast<float4*>(st + (i * CPR + (c ^ (i & (CPR - 1)))) * 16) =
               make_float4(v[4 * q] * alpha, v[4 * q + 1] * alpha, v[4 * q + 2] * alpha, v[4 * q + 3] * alpha);
         }
+      wave_sync();
 #pragma unroll
       for (int jj = 0; jj < 32 / RP; ++jj) {
         const int r = RP * jj + l / LPR, c8 = l % LPR;
@@ -416,6 +422,7 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
           store8(p, (int64_t)(i0 + row) * p.ldo + j0 + col, j0 + col, ya, yb);
         }
       }
+      wave_sync();
     }
 }
 
