@@ -196,3 +196,26 @@ def test_tiny_scales_of_huge_scores(pkg, dev):
     out = pkg.gqa_prefill_attention(q.to(dev), k_new.to(dev), v_new.to(dev), kc.to(dev), vc.to(dev), 0, t, scale=scale)
     err = (out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-2)
     assert float(err.max()) <= 1e-2 and float(err.mean()) <= 2e-3
+
+
+@pytest.mark.parametrize("d,g,t,start", [(d, g, t, s) for d, g, ts in (
+    (64, 1, ((64, 0), (65, 0), (100, 28), (101, 28), (128, 0))), (128, 1, ((65, 63), (127, 1), (129, 0))),
+    (64, 3, ((128, 0), (33, 96))), (64, 5, ((20, 1000), (33, 4063), (33, 4064), (512, 88), (513, 0))), (64, 6, ((40, 600),)),
+    (64, 7, ((17, 520),)), (128, 3, ((12, 500), (13, 500))), (128, 6, ((24, 1000), (25, 1000))),
+    (128, 7, ((31, 1001),))) for t, s in ts])
+def test_few_workgroups_on_both_sides_of_the_16_token_line(pkg, dev, d, g, t, start):
+    """Grids of up to 256 blocks of 16 tokens around the key counts where the two forms change over."""
+    hkv, b, max_len = 2, 2, start + t + 3
+    gen = torch.Generator().manual_seed(1000 * g + t + start)
+    q = torch.randn((b * t, hkv * g * d), generator=gen).to(torch.bfloat16)
+    k_new, v_new = (torch.randn((b * t, hkv * d), generator=gen).to(torch.bfloat16) for _ in range(2))
+    kc, vc = (torch.randn((b, hkv, max_len, d), generator=gen).to(torch.bfloat16) for _ in range(2))
+    kc[:, :, start + t:], vc[:, :, start + t:] = float("inf"), float("nan")  # must not leak in
+    cos, sin = _tables(max_len, d)
+    ref, kc_ref, vc_ref = _reference(q, k_new, v_new, kc, vc, start, t, cos, sin, hkv * g, d ** -0.5)
+    kc_d, vc_d = kc.to(dev), vc.to(dev)
+    out = pkg.gqa_prefill_attention(q.to(dev), k_new.to(dev), v_new.to(dev), kc_d, vc_d, start, t, cos.to(dev),
+                                    sin.to(dev))
+    assert torch.equal(kc_d.cpu(), kc_ref) and torch.equal(vc_d.cpu().view(torch.int16), vc_ref.view(torch.int16))
+    err = (out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-2)
+    assert float(err.max()) <= 1e-2 and float(err.mean()) <= 2e-3

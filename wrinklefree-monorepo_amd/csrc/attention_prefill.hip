@@ -627,18 +627,24 @@ template <int D, int G>
 hipError_t launch_prefill_g(const uint16_t* q, int64_t ldq, const float* rc, const float* rs, const uint16_t* kc,
                             const uint16_t* vc, int64_t max_len, int b, int hkv, int t, int64_t start, float scale,
                             uint16_t* out, int64_t ldo, hipStream_t s) {
-  // Few workgroups (up to one of 16 tokens per CU): the 16-token form where a workgroup's own chain is what the call
-  // takes -- with 3 or more waves on 128-element heads always, else up to 512 keys.  Swept on MI355X over 1 / 3 / 8 kv
-  // heads, 1 / 2 / 4 / 8 query heads each, 20 .. 1000 tokens after 0 or 1000: the line keeps every point within 5% of
-  // the better form (D = 128: 8 x 8 heads, 200 tokens 22.9 against 19.0 us, 1 x 4 heads 512 tokens 24.3 against 21.3;
-  // one CU round more, 8 x 4 heads, 1000 tokens, 39.1 against 49.8 the other way).
-  if constexpr (G >= 2) {
-    const int64_t wg16 = (int64_t)((t + 15) / 16) * hkv * b;
-    if (wg16 <= 256 && ((D == 128 && G >= 3) || start + t <= 512)) {
-      hipLaunchKernelGGL((gqa_prefill16_kernel<D, G>), dim3((t + 15) / 16, hkv, b), dim3(64 * G), 0, s, q, ldq, rc, rs,
-                         kc, vc, max_len, hkv, t, start, scale, out, ldo);
-      return hipGetLastError();
-    }
+  // Few workgroups (up to one of 16 tokens per CU): the 16-token form up to so many keys that a workgroup's own chain
+  // is what the call takes.  Swept on MI355X, both forms, over D 64 / 128, G 1 .. 8, (kv heads, batch) 1 x 1 .. 8 x 1,
+  // 1 x 8 and 3 x 4, 20 (tokens, start) of 16 .. 6033 keys.  The line lies where the 32-token form gets ahead and keeps
+  // every point below 4096 keys within 6% of the better form (16- against 32-token form, one kv head, us):
+  //   G = 1: 128 + 0 tokens 8.5 against 9.1 at D = 64, 10.7 against 11.7 at D = 128; 160 + 0 the other way by 7-12%, as
+  //     is a chunk of fewer tokens behind older keys;
+  //   D = 64: G = 3 loses from 160 keys (8-11%, 17-32% at 256 .. 600); chunks of up to 512 tokens of G = 5 .. 7 win up to
+  //     4096 (64 + 2000 tokens 53.6 against 57.2 at G = 5; 1024 + 0 33.0 against 31.5, and at 6033 keys and 24
+  //     workgroups or more they lose 6-12%); the others lose from 512;
+  //   D = 128: G = 4, 5 and 8 win throughout (33 + 6000 tokens 3, 11 and 0%), G = 6 and 7 up to 1024, G = 2 and 3 up to
+  //     512 (one CU round more, 8 x 4 heads, 1000 tokens, 39.1 against 49.8 the other way).
+  const int64_t keys16 = D == 64 ? (G == 3 ? 128 : G >= 5 && G <= 7 && t <= 512 ? 4096 : 512)
+                                 : (G == 4 || G == 5 || G == 8 ? INT64_MAX : G >= 6 ? 1024 : 512);
+  const int64_t wg16 = (int64_t)((t + 15) / 16) * hkv * b;
+  if (wg16 <= 256 && (G == 1 ? t > 64 && start + t <= 128 : start + t <= keys16)) {
+    hipLaunchKernelGGL((gqa_prefill16_kernel<D, G>), dim3((t + 15) / 16, hkv, b), dim3(64 * G), 0, s, q, ldq, rc, rs,
+                       kc, vc, max_len, hkv, t, start, scale, out, ldo);
+    return hipGetLastError();
   }
   constexpr int QW = G == 1 ? 4 : G == 2 ? 2 : 1;  // three waves or more share each staged K and V tile
   const int64_t nqb = (t + 32 * QW - 1) / (32 * QW), nhb = (int64_t)hkv * b;
