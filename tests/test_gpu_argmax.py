@@ -67,11 +67,24 @@ def test_persistent_head_accumulators(pkg, dev, m, n, k):
 
 
 # plain outputs of 32768 rows and more: persistent from 8 tokens of 2560 (5 waves; 2528 pads to 2560, 3712: 8 waves, the
-# last short), one-shot below, at the edges of the rule and with a ragged last row tile
+# last short), one-shot below and where its workgroups fill whole rounds, with a ragged last row tile
 @pytest.mark.parametrize("m,n,k", [(7, 32768, 2560), (8, 32768, 2560), (8, 32799, 2528), (16, 33009, 3712), (9, 65537, 4096),
                                    (16, 32767, 4096), (17, 32768, 2560)])
 @pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
 def test_plain_head_outputs_match_oracle(pkg, dev, m, n, k, odt):
+    _check_plain_outputs(pkg, dev, m, n, k, odt)
+
+
+# both sides of the persistent form's row counts on 256 CUs: 5 and 7 or more 32-row steps at 2560, more than 4 at 8
+# tokens of longer rows, any at 9
+@pytest.mark.parametrize("m,n,k", [(8, 32769, 2560), (9, 40960, 2560), (9, 40961, 2560), (16, 49152, 2560),
+                                   (16, 49153, 2560), (8, 32768, 3072), (8, 32769, 3072), (9, 32768, 2688)])
+@pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
+def test_plain_outputs_on_both_sides_of_the_persistent_line(pkg, dev, m, n, k, odt):
+    _check_plain_outputs(pkg, dev, m, n, k, odt)
+
+
+def _check_plain_outputs(pkg, dev, m, n, k, odt):
     rng = np.random.default_rng(m + n + k)
     k_pad = -(-k // 128) * 128
     w, a = orc.random_ternary(rng, n, k_pad), np.zeros((m, k_pad), np.int8)

@@ -1006,14 +1006,21 @@ hipError_t launch_modes(const uint8_t* W, int n, int C, const int8_t* A, int m, 
   if (ns.x == nullptr) {
     if (A == nullptr) return hipErrorInvalidValue;
     // many row tiles (the LM head): the persistent form (one token tile), always with a per-lane epilogue (greedy keys,
-    // accumulators), for plain outputs where the one-shot form's activation staging costs more than its whole-line
-    // stores save: from 8 tokens of 2560 or more (cold weights on MI355X, one-shot against persistent: 128256 x 4096
-    // at M = 8 36.3 -> 27.2 us, M = 16 45.0 -> 29.5; x 2560 28.6 -> 26.3 and 30.2 -> 26.9, but M = 4 21.6 -> 25.7;
-    // 32768 x 2048 at M = 16 6.8 -> 9.3, 49152 x 640 7.0 -> 12.1)
+    // accumulators); for plain outputs from 8 tokens of 2560 on, where the one-shot form's activation staging costs more
+    // than its whole-line stores save, unless its workgroups come out in few whole rounds: of 64 rows at 2560 (two
+    // persistent steps a round, ahead up to three rounds), of 128 rows at 8 tokens of more (four steps, ahead in one).
+    // Cold weights on MI355X, one-shot against persistent, bf16 outputs, us:
+    //   2560 at M = 8 / 16: 32768 rows 9.9 / 10.3 against 10.7 / 11.0, 33000 12.8 / 13.2 against 12.2 / 12.2, 49152 14.1 /
+    //     14.8 against 14.7 / 15.4, 49153 16.1 / 16.6 against 15.5 / 15.9, 128256 33.0 / 34.4 against 27.6 / 28.3;
+    //   3072 and 4096 at M = 8: 32768 rows 9.6 and 10.9 against 10.2 and 11.0, 33000 14.8 and 16.1 against 11.5 and 12.2;
+    //     at M = 9 32768 rows 11.7 and 12.8 against 10.3 and 11.2; 128256 x 4096 at M = 16 44.2 against 29.6;
+    //   M = 4: 128256 x 2560 21.6 against 25.7; shorter rows: 32768 x 2048 at M = 16 6.8 against 9.3.
     if constexpr (MR <= 16) {
       const bool lanes = e.amax || e.acc_out || !e.out;
-      if (GLUE == 0 && (lanes || (m >= 8 && C >= 40)) && !e.bias && !e.res && e.nseg == 1 && n >= kPersistMinRows) {
-        const hipError_t st = launch_persist(W, n, C, A, m, lda, e, cu_count(), s);
+      const int cus = cu_count(), steps = ((n + 31) / 32 + cus - 1) / cus;  // 32-row steps of a persistent workgroup
+      const bool plain = m >= 8 && (C > 40 ? m > 8 || steps > 4 : C == 40 && (steps > 6 || steps == 5));
+      if (GLUE == 0 && (lanes || plain) && !e.bias && !e.res && e.nseg == 1 && n >= kPersistMinRows) {
+        const hipError_t st = launch_persist(W, n, C, A, m, lda, e, cus, s);
         if (st != hipErrorNotSupported) return st;
       }
     }
