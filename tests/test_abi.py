@@ -273,6 +273,19 @@ def test_fusion_predicates_match_the_entry_points(pkg):
                 m, h, k)
 
 
+def test_fused_norm_is_preferred_where_it_measures_faster(pkg):
+    """(M, K, rows) on both sides of the line between the fused norm + linear and two launches, a point each of the
+    sweep that the rule states."""
+    fused = [(1, 4096, 49152), (1, 576, 32768), (2, 2048, 128256), (2, 1664, 65536), (2, 4096, 49152), (3, 4096, 32768),
+             (4, 2048, 32768), (5, 2560, 32768), (6, 2048, 32768), (8, 4096, 32768), (16, 4096, 6144)]
+    two = [(1, 4096, 65536), (2, 1536, 65536), (2, 2176, 65536), (2, 4096, 128256), (3, 576, 49152), (3, 4096, 40960),
+           (4, 3072, 40960), (6, 1024, 32768), (8, 2560, 32768), (8, 3072, 40960), (16, 4096, 32768), (16, 576, 128256)]
+    for m, k, n in fused:
+        assert pkg.rmsnorm_linear_preferred(m, k, n, (k + 127) // 128 * 128), (m, k, n)
+    for m, k, n in two:
+        assert not pkg.rmsnorm_linear_preferred(m, k, n, (k + 127) // 128 * 128), (m, k, n)
+
+
 def test_rmsnorm_linear_glu_argument_errors(pkg):
     vp = ctypes.c_void_p
 

@@ -501,12 +501,20 @@ def rmsnorm_linear_glu_supported(m: int, h: int, k: int) -> bool:
 
 
 def rmsnorm_linear_preferred(m: int, h: int, n: int, k: int, gamma_bytes: int = 2) -> bool:
-    """Whether the fused launch is the faster choice.  Its workgroups each repeat the norm, which up to some 32768
-    output rows costs less than the separate quantiser launch it replaces (measured on MI355X at the Llama-3-8B,
-    BitNet-2B and SmolLM2 decode shapes) and on a vocabulary's rows more: quantiser and linear against fused, cold
-    weights, 128256 x 4096 at M = 1 / 8 / 16 25 / 33 / 35 us against 30 / 50 / 86, 49152 x 640 at M = 3 / 16 7.3 / 9.7
-    against 12.8 / 35; 32768 x 2048 at M = 2 / 4 10.9 / 9.7 against 8.4 / 8.5, M = 8 9.8 against 10.3."""
-    wide = n >= 65536 or (n >= 32768 and m * n >= 147456)
+    """Whether the fused launch is the faster choice.  Each of its workgroups repeats the norm, which costs less than
+    the separate quantiser launch while one round of them (32768 output rows on 256 CUs) covers the outputs, and more
+    on a vocabulary's rows.  Swept on MI355X, cold weights, K of 576 to 4096, 16384 to 128256 rows (fused against
+    quantiser and linear, us): 3 to 8 tokens cross over behind 32768 rows (M = 3, 32768 against 40960 rows of 4096 12.5
+    / 14.6 and 19.5 / 16.9), at them from 5 tokens on K <= 1024 and from 6 on K <= 1536 and 2176 to 2560 (M = 6, 32768
+    rows of 1024 9.9 / 7.7, of 2560 15.8 / 14.5, of 2048 10.1 / 10.2, of 3072 12.1 / 14.5); more than 8 at them (M = 16,
+    32768 x 4096 23.3 / 17.8; fewer rows are not told apart here); one token by 65536 rows (x 4096 17.4 / 16.8, x 2560
+    19.1 / 14.6); two too (x 4096 22.7 / 19.2), but not on K of 1664 to 2048, where the two-token linear itself is slow
+    (128256 x 2048 25.1 / 30.5; x 1536 23.5 / 20.2)."""
+    mid = 1536 < k <= 2048
+    if m <= 2:
+        wide = n >= 65536 and not (m == 2 and mid)
+    else:
+        wide = n > 32768 or (n == 32768 and (m > 8 or (m > 4 and k <= 1024) or (m > 5 and k <= 2560 and not mid)))
     return not wide and rmsnorm_linear_supported(m, h, k, gamma_bytes)
 
 
