@@ -120,6 +120,14 @@ def test_pack_codes_around_half_a_scale(pkg, dev, dtype, n, k):
         assert np.array_equal(qw.cpu().numpy(), ref), s
 
 
+# the elements of a thread: none for most, one, two (the last of the short form), three, 16 and one more
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("numel", [1, 255, 262144, 524288, 524289, 786431, 4194304, 4194305])
+def test_absmean_sums_in_one_order_at_every_length(pkg, dev, dtype, numel):
+    w = torch.from_numpy((np.random.default_rng(numel).standard_normal(numel) * 0.05).astype(np.float32)).to(dtype)
+    assert np.float32(pkg.absmean_scale(w.to(dev)).item()) == orc.absmean_scale_device_order(w.float().numpy())
+
+
 def test_absmean_tiny_weights(pkg, dev):
     w = torch.full((8, 128), 1e-9, device=dev)
     assert pkg.absmean_scale(w).item() == 1.0
