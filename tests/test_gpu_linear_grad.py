@@ -70,6 +70,27 @@ def test_non_finite_gradients_reach_the_products(pkg, dev):
         assert torch.allclose(got[fine].double(), want[fine], rtol=0, atol=1e-5 * float(want[fine].abs().max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("scale", [0.02, 2.0 ** -20, -0.3, 1.5, 3e-40, 0.0])
+@pytest.mark.parametrize("n", [72, 4040])
+def test_grad_x_is_bounded_by_its_result_not_by_the_unscaled_sum(pkg, dev, dtype, scale, n):
+    """Gradients whose sum against the ternary weight (standard deviation sd) leaves fp32's range before the weight
+    scale brings it back, and scales that are negative, above 1, subnormal or zero, summed whole and in parts."""
+    ops, m, k = pkg.ops, 40, 264
+    g = torch.Generator(device=dev).manual_seed(n)
+    qw, _ = ops.pack_ternary_i2s(torch.randn((n, k), generator=g, device=dev), k_pad=384)
+    t = ops.unpack_i2s(qw)[:, :k].double()
+    sd = 1.2e38 if abs(scale) < 1 else 3e37
+    gy = (torch.randn((m, n), generator=g, device=dev) * (sd / float(t.pow(2).sum(0).mean().sqrt()))).to(dtype)
+    s = torch.full((1,), scale, device=dev)
+    sums = gy.double() @ t
+    assert abs(scale) > 1 or float(sums.abs().max()) > torch.finfo(torch.float32).max
+    got, want = ops.linear_grad_x(qw, s, gy, k, torch.float32), sums * s.double()
+    # (a subnormal result is rounded to 2^-149)
+    assert torch.isfinite(got).all()
+    assert float((got.double() - want).norm()) <= 1e-6 * float(want.norm()) + 2.0 ** -149 * (m * k) ** 0.5
+
+
 def test_gradients_of_gradients_and_batched_gradients_keep_working(pkg, dev):
     """create_graph and is_grads_batched go through the torch products that autograd and vmap see through."""
     torch.manual_seed(5)

@@ -157,10 +157,19 @@ __global__ __launch_bounds__(256) void codes_t_kernel(const int8_t* __restrict__
   }
 }
 
-// I2_S codes of W[n][k] as bf16 {-1, 0, 1} dst[k][n], rows of np elements (n >= N: zeros).  One 128-weight block
-// of 64 rows per workgroup.
+// The weight scale's power of two, 2^-126 at least; 1 for a scale that is not finite.  The weight codes
+// carry it (exact in bf16), so the sums of a gradient run at the size of its result, and the epilogue's factor is what
+// is left of the scale: the same bits, without overflow where only the unscaled sum leaves fp32's range.
+__device__ __forceinline__ float scale_unit(float s) {
+  const uint32_t e = __float_as_uint(s) & 0x7f800000u;
+  return e == 0x7f800000u ? 1.0f : __uint_as_float(e ? e : 0x00800000u);
+}
+
+// I2_S codes of W[n][k] as bf16 {-u, 0, u}, u = scale_unit(scale), dst[k][n], rows of np elements (n >= N: zeros).
+// One 128-weight block of 64 rows per workgroup.
 __global__ __launch_bounds__(256) void weight_codes_t_kernel(const uint8_t* __restrict__ qw, int64_t row_bytes,
                                                              int64_t N, int64_t K, int64_t np,
+                                                             const float* __restrict__ scale,
                                                              uint16_t* __restrict__ dst) {
   __shared__ __attribute__((aligned(4))) uint8_t tile[64][36];
   const int64_t n0 = (int64_t)blockIdx.x * 64, b = blockIdx.y;
@@ -172,6 +181,7 @@ __global__ __launch_bounds__(256) void weight_codes_t_kernel(const uint8_t* __re
     t[0] = n < N ? w.x : 0x55555555u;
     t[1] = n < N ? w.y : 0x55555555u;
   }
+  const float unit = scale_unit(scale[0]);
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < 4; ++it) {
@@ -183,7 +193,7 @@ __global__ __launch_bounds__(256) void weight_codes_t_kernel(const uint8_t* __re
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int code = (tile[8 * ch + e][j] >> sh) & 3;
-      o.h[e] = (uint16_t)(__float_as_uint((float)(code - 1)) >> 16);
+      o.h[e] = (uint16_t)(__float_as_uint((float)(code - 1) * unit) >> 16);
     }
     *reinterpret_cast<uint4*>(dst + k * np + n) = o.q4;
   }
@@ -206,13 +216,19 @@ struct GradGemm {
   int stages;          // of BK elements, all splits together
   int full;            // the first `full` tiles are summed by one workgroup each,
   int nsplit;          // the others by nsplit: split s takes stages [s * per, ...), per = ceil(stages / nsplit)
-  const float* alpha;  // device scalar or null (1)
+  const float* alpha;  // device scalar, of which the B rows carry scale_unit, or null (1)
   float* parts;        // fp32 partial tiles [tiles past full][nsplit][BI][BJ]
   void* out;           // [I][ldo] in out_dtype
   int out_dtype;
   int64_t ldo;
   bool vec;            // rows of out 16-byte aligned
 };
+
+__device__ __forceinline__ float alpha_of(const GradGemm& p) {
+  if (!p.alpha) return 1.0f;
+  const float s = p.alpha[0];
+  return __fdiv_rn(s, scale_unit(s));  // (exact)
+}
 
 __device__ __forceinline__ void store1(const GradGemm& p, int64_t off, float y) {
   if (p.out_dtype == WFB_F32) reinterpret_cast<float*>(p.out)[off] = y;
@@ -386,7 +402,7 @@ __global__ __launch_bounds__(64 * WI * WJ) __attribute__((amdgpu_waves_per_eu(WP
   constexpr int WPB = SZ / ST;                     // waves whose staging fits one buffer
   static_assert(TJ % TS == 0 && WPB >= 1 && 2 * WPB >= W, "staging fits the two operand buffers");
   uint8_t* st = w < WPB ? lds0 + w * ST : lds1 + (w - WPB) * ST;
-  const float alpha = whole && p.alpha ? p.alpha[0] : 1.0f;
+  const float alpha = whole ? alpha_of(p) : 1.0f;
   constexpr int LPR = CPR / 2, RP = 64 / LPR;
   float* const part = whole ? nullptr : p.parts + (int64_t)u * (BI * BJ);
   auto wave_sync = [] {  // orders the wave's LDS accesses for the compiler (the LDS keeps a wave's order by itself)
@@ -441,7 +457,7 @@ __global__ __launch_bounds__(256) void grad_reduce_kernel(GradGemm p, int bi, in
     a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
     b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
   }
-  const float alpha = p.alpha ? p.alpha[0] : 1.0f;
+  const float alpha = alpha_of(p);
   store8(p, (int64_t)row * p.ldo + col, col, make_float4(a.x * alpha, a.y * alpha, a.z * alpha, a.w * alpha),
          make_float4(b.x * alpha, b.y * alpha, b.z * alpha, b.w * alpha));
 }
@@ -571,7 +587,7 @@ hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t
   uint16_t* gp = reinterpret_cast<uint16_t*>(ws + align256(2 * k * np));
   float* parts = reinterpret_cast<float*>(ws + align256(2 * k * np) + align256(2 * P * m * np));
   hipLaunchKernelGGL(weight_codes_t_kernel, dim3((unsigned)(np / 64), (unsigned)((k + 127) / 128)), dim3(256), 0, s, qw,
-                     k_pad / 4, n, k, np, wt);
+                     k_pad / 4, n, k, np, w_scale, wt);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   GradGemm p{};
