@@ -81,8 +81,9 @@ def _kernel_grads(gy: torch.Tensor, in_features: int, *saved: torch.Tensor) -> b
         return False
     if type(gy) not in (torch.Tensor, nn.Parameter) or gy.is_neg():
         return False
-    if any(not t.is_contiguous() or t.is_neg() for t in saved):
-        return False
+    for t in saved:
+        if t.is_neg() or not t.is_contiguous():
+            return False
     return linear_grad_supported(gy, in_features)
 
 

@@ -688,7 +688,7 @@ def linear_grad_supported(grad: torch.Tensor, in_features: int) -> bool:
 
 def _grad_workspace(m: int, n: int, k: int, dt: int, which: int, dev: torch.device) -> torch.Tensor:
     size = ctypes.c_int64(0)
-    ptr = ctypes.cast(ctypes.byref(size), ctypes.c_void_p)
+    ptr = ctypes.addressof(size)
     _lib.call("wfb_linear_grad_workspace", m, n, k, dt, ptr if which == 0 else None, ptr if which == 1 else None)
     return torch.empty(size.value, dtype=torch.uint8, device=dev)
 
