@@ -379,8 +379,11 @@ int wfb_linear_i2s_glu(const uint8_t* qweight, int64_t n, int64_t k, const int8_
  * fp32 and the sums are fp32.  g: fp32 / bf16 / fp16 [M, N], row stride ldg; w_scale_dev, a_scale: fp32 on the
  * device; out: fp32 / bf16 / fp16, row stride ldo.  bias_out [N] of type bias_dtype (or NULL) takes sum_m g[m, n],
  * summed in fp32.  work: 16-byte aligned device memory of at least the bytes
- * wfb_linear_grad_workspace reports (host only, no GPU work).  M, N, K >= 1 and below 2^20 each. */
+ * wfb_linear_grad_workspace reports (host only, no GPU work).  M, N, K >= 1 and below 2^20 each.
+ * wfb_linear_grad_plan (host only) tells how the products are cut, five values each: rows and columns of an output
+ * tile, tiles, how many of them one workgroup sums, and the parts that the sum of each other one is cut into. */
 int wfb_linear_grad_workspace(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* bytes_x, int64_t* bytes_w);
+int wfb_linear_grad_plan(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* plan_x, int64_t* plan_w);
 int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const uint8_t* qweight,
                       int64_t k, int64_t k_pad, const float* w_scale_dev, void* out, int out_dtype, int64_t ldo,
                       void* work, void* stream);

@@ -306,6 +306,55 @@ def test_rmsnorm_linear_glu_argument_errors(pkg):
     assert st(m=0) == 0
 
 
+def test_gradient_argument_errors(pkg):
+    vp = ctypes.c_void_p
+
+    def gx(g=16, g_dt=1, ldg=64, m=4, n=64, qw=16, k=100, k_pad=128, sc=16, out=16, out_dt=0, ldo=100, work=16):
+        return pkg._lib.status("wfb_linear_grad_x", vp(g), g_dt, ldg, m, n, vp(qw), k, k_pad, vp(sc), vp(out), out_dt,
+                               ldo, vp(work), None)
+
+    def gw(g=16, g_dt=1, ldg=64, m=4, n=64, act=16, lda=128, sc=16, k=100, out=16, out_dt=0, ldo=100, b=None, b_dt=0,
+           work=16):
+        return pkg._lib.status("wfb_linear_grad_w", vp(g), g_dt, ldg, m, n, vp(act), lda, vp(sc), k, vp(out), out_dt,
+                               ldo, b, b_dt, vp(work), None)
+
+    for f in (gx, gw):
+        assert f(g_dt=3) == -1 and "bad gradient dtype" in pkg._lib.last_error()
+        for size in ("m", "n", "k"):
+            for bad in (0, 1 << 20):
+                assert f(**{size: bad}) == -1 and "outside 1..2^20-1" in pkg._lib.last_error()
+        for ptr in ("g", "sc", "out", "work"):
+            assert f(**{ptr: None}) == -1 and "null pointer" in pkg._lib.last_error()
+        assert f(out_dt=3) == -1 and "bad output dtype" in pkg._lib.last_error()
+        assert f(ldg=63) == -1 and f(ldg=1 << 21) == -1 and f(ldo=99) == -1 and "row strides" in pkg._lib.last_error()
+        assert f(work=24) == -1 and "16-byte aligned" in pkg._lib.last_error()
+    assert gx(qw=None) == -1 and gw(act=None) == -1 and "null pointer" in pkg._lib.last_error()
+    assert gx(k_pad=64) == -1 and gx(k=60, k_pad=64) == -1 and gx(qw=20) == -1
+    assert "packed rows" in pkg._lib.last_error()
+    assert gw(lda=99) == -1 and "activation row stride" in pkg._lib.last_error()
+    assert gw(b=vp(16), b_dt=3) == -1 and "bad bias dtype" in pkg._lib.last_error()
+    st = pkg._lib.status
+    for fn in ("wfb_linear_grad_workspace", "wfb_linear_grad_plan"):
+        assert st(fn, 4, 64, 100, 3, None, None) == -1 and st(fn, 0, 64, 100, 1, None, None) == -1
+        assert st(fn, 4, 64, 100, 1, None, None) == 0
+
+
+def test_norm_gradient_argument_errors(pkg):
+    vp = ctypes.c_void_p
+
+    def st(x=16, x_dt=1, gamma=16, g_dt=1, g=16, m=4, h=64, gx=16, gg=16, gg_dt=1, work=16):
+        return pkg._lib.status("wfb_rmsnorm_grad", vp(x), x_dt, vp(gamma), g_dt, vp(g), 1e-6, m, h, vp(gx), vp(gg),
+                               gg_dt, vp(work), None)
+
+    assert st(x_dt=3) == -1 and st(g_dt=3) == -1 and st(gg_dt=3) == -1 and "bad dtype" in pkg._lib.last_error()
+    assert st(h=60) == -1 and st(h=0) == -1 and st(h=16392) == -1 and "multiple of 8" in pkg._lib.last_error()
+    assert st(m=-1) == -1
+    assert st(x=None) == -1 and st(gamma=None) == -1 and st(g=None) == -1 and st(work=None) == -1
+    assert st(gx=None, gg=None) == -1 and "null pointer" in pkg._lib.last_error()
+    assert st(g=8) == -1 and st(gx=8) == -1 and st(work=8) == -1 and "aligned" in pkg._lib.last_error()
+    assert st(m=0, gg=None) == 0
+
+
 def test_linear_glu_argument_errors(pkg):
     vp = ctypes.c_void_p
 

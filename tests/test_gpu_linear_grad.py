@@ -7,6 +7,8 @@ at most about sqrt(3 C / 16) roundings of 2^-24 (three planes, 16 terms per matr
 g * a_scale and the result's own: below 1e-6 for C <= 2048 (measured 0.3-4e-7); 16-bit outputs are the fp32 result
 rounded once, bit for bit."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -36,6 +38,57 @@ def test_linear_grads_match_float64(pkg, dev, m, n, k, dtype):
     for out in (torch.bfloat16, torch.float16):
         assert torch.equal(ops.linear_grad_x(qw, scale, gy, k, out), gx.to(out))
         assert torch.equal(ops.linear_grad_w(codes, a_scale, gy, k, out), gw.to(out))
+
+
+# One case for every form that the plan picks: each tile size, its tiles summed whole, all of them in parts, or only
+# those past the last full round of workgroups; every edge ragged.
+_FORMS = [
+    ("x", torch.bfloat16, (70, 84, 69), (64, 128, "whole")), ("x", torch.bfloat16, (77, 787, 78), (64, 128, "parts")),
+    ("x", torch.bfloat16, (7254, 74, 799), (128, 128, "whole")),
+    ("x", torch.bfloat16, (962, 1697, 1163), (128, 128, "parts")),
+    ("x", torch.bfloat16, (3867, 1265, 2116), (128, 128, "rest")),
+    ("x", torch.bfloat16, (5831, 68, 2087), (256, 256, "whole")),
+    ("x", torch.bfloat16, (1421, 5384, 1960), (256, 256, "parts")),
+    ("x", torch.bfloat16, (3545, 1512, 4821), (256, 256, "rest")),
+    ("x", torch.float32, (70, 84, 69), (64, 128, "whole")), ("x", torch.float32, (72, 211, 72), (64, 128, "parts")),
+    ("x", torch.float32, (1691, 493, 4781), (64, 128, "rest")),
+    ("x", torch.float32, (2382, 78, 3339), (128, 256, "whole")),
+    ("x", torch.float32, (1374, 1547, 1960), (128, 256, "parts")),
+    ("x", torch.float32, (3122, 325, 5264), (128, 256, "rest")),
+    ("w", torch.bfloat16, (70, 84, 69), (64, 128, "whole")), ("w", torch.bfloat16, (226, 72, 71), (64, 128, "parts")),
+    ("w", torch.bfloat16, (479, 3118, 2617), (64, 128, "rest")),
+    ("w", torch.bfloat16, (75, 4729, 1722), (128, 256, "whole")),
+    ("w", torch.bfloat16, (1541, 1266, 2224), (128, 256, "parts")),
+    ("w", torch.bfloat16, (344, 6602, 2551), (128, 256, "rest")),
+]
+
+
+@pytest.mark.parametrize("which,dtype,size,form", _FORMS)
+def test_every_tile_form_matches_float64(pkg, dev, which, dtype, size, form):
+    ops, (m, n, k) = pkg.ops, size
+    plan = (ctypes.c_int64 * 5)()
+    ptr = ctypes.addressof(plan)
+    pkg._lib.call("wfb_linear_grad_plan", m, n, k, 0 if dtype == torch.float32 else 1, ptr if which == "x" else None,
+                  ptr if which == "w" else None)
+    bi, bj, tiles, full, parts = plan
+    how = "whole" if full == tiles else "rest" if full else "parts"
+    assert (bi, bj, how) == form and (parts > 1) == (how != "whole")
+    g = torch.Generator(device=dev).manual_seed(m)
+    rand = lambda *s: torch.randn(s, generator=g, device=dev)  # noqa: E731
+    k_pad = (k + 127) // 128 * 128
+    gy = rand(m, n).to(dtype)
+    # sums of C terms, P planes of 16 terms per matrix instruction: that many roundings of 2^-24, and two more
+    planes, terms = (1 if dtype == torch.bfloat16 else 3, n) if which == "x" else (3, m)
+    tol = 2.0 ** -24 * ((planes * terms / 16) ** 0.5 + 2)
+    if which == "x":
+        qw, scale = ops.pack_ternary_i2s(rand(n, k) * 0.02, k_pad=k_pad)
+        got = ops.linear_grad_x(qw, scale, gy, k, torch.float32)
+        want = (gy.double() @ ops.unpack_i2s(qw)[:, :k].double()) * scale.double()
+    else:
+        codes, a_scale = ops.quantize_activations_i8_per_token(rand(m, k) * (1 + rand(m, 1).abs()), k_pad=k_pad)
+        got = ops.linear_grad_w(codes, a_scale, gy, k, torch.float32)
+        want = (gy.double() * a_scale.double()[:, None]).t().contiguous() @ codes[:, :k].double()
+    assert _rel(got, want) <= tol
 
 
 @pytest.mark.parametrize("m", [520, 1030])

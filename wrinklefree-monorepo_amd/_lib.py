@@ -38,6 +38,7 @@ SIGNATURES = {
     "wfb_pack_i2s": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp],
     "wfb_unpack_i2s": [_vp, _i64, _i64, _vp, _vp],
     "wfb_linear_grad_workspace": [_i64, _i64, _i64, _int, _vp, _vp],
+    "wfb_linear_grad_plan": [_i64, _i64, _i64, _int, _vp, _vp],
     "wfb_linear_grad_x": [_vp, _int, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _int, _i64, _vp, _vp],
     "wfb_linear_grad_w": [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _int, _i64, _vp, _int, _vp, _vp],
     "wfb_rmsnorm_grad": [_vp, _int, _vp, _int, _vp, _f32, _i64, _i64, _vp, _vp, _int, _vp, _vp],

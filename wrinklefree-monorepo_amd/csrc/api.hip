@@ -228,6 +228,17 @@ int wfb_linear_grad_workspace(int64_t m, int64_t n, int64_t k, int g_dtype, int6
   return ok();
 }
 
+int wfb_linear_grad_plan(int64_t m, int64_t n, int64_t k, int g_dtype, int64_t* plan_x, int64_t* plan_w) {
+  if (const int st = grad_sizes("wfb_linear_grad_plan", m, n, k, g_dtype)) return st;
+  int64_t p[5];
+  for (int64_t* out : {plan_x, plan_w}) {
+    if (!out) continue;
+    wfb::grad_plan(out == plan_x, m, n, k, g_dtype, p);
+    std::copy(p, p + 5, out);
+  }
+  return ok();
+}
+
 int wfb_linear_grad_x(const void* g, int g_dtype, int64_t ldg, int64_t m, int64_t n, const uint8_t* qweight, int64_t k,
                       int64_t k_pad, const float* w_scale_dev, void* out, int out_dtype, int64_t ldo, void* work,
                       void* stream) {

@@ -577,6 +577,13 @@ int64_t grad_w_workspace(int64_t m, int64_t n, int64_t k) {
          part_bytes(plan(3, n, k, m));
 }
 
+void grad_plan(bool of_x, int64_t m, int64_t n, int64_t k, int gdt, int64_t (&out)[5]) {
+  const Plan pl = of_x ? plan(grad_x_planes(gdt), m, k, n) : plan(3, n, k, m);
+  const Variant& v = kVariants[pl.variant];
+  const int64_t o[5] = {v.bi, v.bj, pl.tiles, pl.full, pl.nsplit};
+  std::copy(o, o + 5, out);
+}
+
 hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const uint8_t* qw, int64_t k,
                          int64_t k_pad, const float* w_scale, void* out, int odt, int64_t ldo, void* work,
                          hipStream_t s) {

@@ -481,6 +481,8 @@ hipError_t launch_unpack_i2s(const uint8_t* qw, int64_t n, int64_t k, int8_t* ou
 // Straight-through gradients (grad.hip); workspace bytes of each.
 int64_t grad_x_workspace(int64_t m, int64_t n, int64_t k, int gdt);
 int64_t grad_w_workspace(int64_t m, int64_t n, int64_t k);
+// {tile rows, tile columns, tiles, tiles summed by one workgroup, parts of each other tile} of grad_x / grad_w
+void grad_plan(bool of_x, int64_t m, int64_t n, int64_t k, int gdt, int64_t (&out)[5]);
 hipError_t launch_grad_x(const void* g, int gdt, int64_t ldg, int64_t m, int64_t n, const uint8_t* qw, int64_t k,
                          int64_t k_pad, const float* w_scale, void* out, int odt, int64_t ldo, void* work,
                          hipStream_t s);
