@@ -145,6 +145,25 @@ def test_dense_head_argmax_matches_torch(pkg, dev, m, n, h, xdt, wdt):
     assert torch.equal(pkg.lm_head_argmax(x.to(dev), w.to(dev), g.to(dev), eps=1e-5), tok)
 
 
+# two and one row groups at once with a ragged vocabulary, fewer tokens than the form holds, rows of one chunk and with
+# chunks left over after the batches of 32
+@pytest.mark.parametrize("m,n,h", [(1, 1001, 2056), (1, 17, 8), (2, 1001, 2056), (3, 17, 8), (4, 129, 576),
+                                   (5, 3001, 1000), (8, 777, 2048), (11, 100, 1288), (16, 4099, 1024)])
+def test_bf16_head_sums_in_fp32(pkg, dev, m, n, h):
+    """Rows of +-1 under eps 0 have the norm x * gamma exactly, so the logits stand against float64 products of the very
+    same bf16 rows.  Bound: an element passes 4 two-element dot products, h / 64 running sums and 3 lane sums, each
+    within 2^-23 of the sum of magnitudes."""
+    gen = torch.Generator().manual_seed(m + n + h)
+    x = (torch.randint(0, 2, (m, h), generator=gen) * 2 - 1).to(torch.bfloat16)
+    w = (torch.randn((n, h), generator=gen) * 0.02).to(torch.bfloat16)
+    g = (1 + 0.1 * torch.randn(h, generator=gen)).to(torch.bfloat16)
+    y = x.double() * g.double()
+    tok, logits = pkg.lm_head_argmax(x.to(dev), w.to(dev), g.to(dev), eps=0.0, return_logits=True)
+    bound = (4 + -(-h // 64) + 3) * 2.0 ** -23 * (y.abs() @ w.double().abs().T)
+    assert bool(((logits.cpu().double() - y @ w.double().T).abs() <= bound).all())
+    assert np.array_equal(tok.cpu().numpy(), _first_argmax(logits.cpu().numpy()))
+
+
 def test_dense_head_argmax_ties_pick_first(pkg, dev):
     gen = torch.Generator().manual_seed(1)
     w = torch.randn((300, 128), generator=gen) * 0.01
