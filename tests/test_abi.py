@@ -371,6 +371,15 @@ def test_linear_glu_argument_errors(pkg):
     assert st(m=0) == 0
 
 
+def test_device_guard_follows_the_current_device(pkg, monkeypatch):
+    """Calls enter a device guard exactly when the tensors' device is not the current one."""
+    for current, guarded in ((0, False), (1, True)):
+        monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda c=current: c)
+        ctx = pkg.ops._on(torch.device("cuda:0"))
+        assert isinstance(ctx, torch.cuda.device) == guarded
+        assert not guarded or ctx.idx == 0
+
+
 def test_fused_op_weight_cache(pkg):
     """The fused reference ops' weight concatenations (host logic, CPU tensors): a single weight is used as it
     is (no copy), a set is concatenated once and reused until a weight changes in place, and the cache holds

@@ -128,6 +128,28 @@ def test_absmean_sums_in_one_order_at_every_length(pkg, dev, dtype, numel):
     assert np.float32(pkg.absmean_scale(w.to(dev)).item()) == orc.absmean_scale_device_order(w.float().numpy())
 
 
+def test_calls_run_on_the_current_stream(pkg, dev):
+    """On a side stream held up by a spin, the calls wait behind it and read what it leaves."""
+    rng = np.random.default_rng(9)
+    w = torch.from_numpy((rng.standard_normal((576, 640)) * 0.02).astype(np.float32)).to(dev)
+    x = torch.from_numpy(rng.standard_normal((5, 640)).astype(np.float32)).to(dev)
+    qw, scale = pkg.pack_ternary_i2s(w)
+    q, a = pkg.quantize_activations_i8_per_token(x)
+    want = pkg.bitnet_linear(qw, q, scale, a_scale=a, out_dtype=torch.float32)
+    late = torch.zeros_like(x)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        assert pkg.ops._stream(dev) == side.cuda_stream
+        torch.cuda._sleep(20_000_000)  # some 10 ms
+        late.copy_(x)
+        q2, a2 = pkg.quantize_activations_i8_per_token(late)
+        got = pkg.bitnet_linear(qw, q2, scale, a_scale=a2, out_dtype=torch.float32)
+    assert pkg.ops._stream(dev) == torch.cuda.current_stream().cuda_stream != side.cuda_stream
+    side.synchronize()
+    assert torch.equal(q2, q) and torch.equal(got, want)
+
+
 def test_absmean_tiny_weights(pkg, dev):
     w = torch.full((8, 128), 1e-9, device=dev)
     assert pkg.absmean_scale(w).item() == 1.0
