@@ -161,7 +161,7 @@ class _SubLNBitLinearSTE(torch.autograd.Function):
             if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
                 # gradient at the norm's output (identity through the quantiser), then the norm's own
                 g_norm = linear_grad_x(qweight, wscale, gy, kin, torch.float32)
-                gx, gg = rmsnorm_grad(x2.detach(), gamma.detach(), g_norm, eps, *ctx.needs_input_grad[:2])
+                gx, gg = rmsnorm_grad(x2, gamma, g_norm, eps, *ctx.needs_input_grad[:2])
             return gx, gg, gw, gb, None, None
         g = gy.to(torch.float32).contiguous()
         gx = gg = gw = gb = None
