@@ -145,10 +145,11 @@ def test_dense_head_argmax_matches_torch(pkg, dev, m, n, h, xdt, wdt):
     assert torch.equal(pkg.lm_head_argmax(x.to(dev), w.to(dev), g.to(dev), eps=1e-5), tok)
 
 
-# two and one row groups at once with a ragged vocabulary, fewer tokens than the form holds, rows of one chunk and with
+# two and one row groups at once (the last three: one for several tokens) with a ragged vocabulary, fewer tokens than the form holds, rows of one chunk and with
 # chunks left over after the batches of 32
 @pytest.mark.parametrize("m,n,h", [(1, 1001, 2056), (1, 17, 8), (2, 1001, 2056), (3, 17, 8), (4, 129, 576),
-                                   (5, 3001, 1000), (8, 777, 2048), (11, 100, 1288), (16, 4099, 1024)])
+                                   (5, 3001, 1000), (8, 777, 2048), (11, 100, 1288), (16, 4099, 1024),
+                                   (2, 32777, 4096), (3, 32777, 2560), (4, 40969, 4096)])
 def test_bf16_head_sums_in_fp32(pkg, dev, m, n, h):
     """Rows of +-1 under eps 0 have the norm x * gamma exactly, so the logits stand against float64 products of the very
     same bf16 rows.  Bound: an element passes 4 two-element dot products, h / 64 running sums and 3 lane sums, each

@@ -17,11 +17,11 @@
 // accumulation, a DPP sum over the 8 lanes; each wave covers 16 rows = one workspace slot.  bf16 rows against a
 // bf16 embedding (the normalised rows are bf16 values then) are kept as bf16 in LDS and multiplied two elements per
 // instruction (v_dot2c_f32_bf16, exact products, fp32 sums), and from two tokens on each LDS read serves a wave's two
-// groups of 8 rows.  One token is bound by the weight stream; at more, widening, multiplying and adding each element
-// of each token by itself took 9 vector operations a weight at 4 tokens, and the rows twice the LDS bytes.  Whole
-// call with the finalize, before and after: 128256 x 2560 at M = 2 134 -> 119 us, M = 4 174 -> 131 (5.0 TB/s), M = 6
-// 262 -> 143; 128256 x 1024 at M = 16 255 -> 136; 49152 x 576 at M = 8 38 -> 31; M = 1 unchanged (its two row
-// groups stay one after the other: together they took 66 instead of 56 us at 33333 x 4096).
+// groups of 8 rows, but for the shapes at launch_head_t.  One token is bound by the weight stream; at more, widening,
+// multiplying and adding each element of each token by itself took 9 vector operations a weight at 4 tokens, and the
+// rows twice the LDS bytes.  Whole call with the finalize, cold weights, before and after: 128256 x 2560 at M = 2 139 ->
+// 126 us, M = 4 163 -> 138, M = 6 260 -> 147; 128256 x 1024 at M = 16 256 -> 135; 49152 x 576 at M = 8 38 -> 32; M = 1
+// unchanged (its two row groups stay one after the other: together they took 68.6 instead of 60.7 us at 33333 x 4096).
 #include "wfb_common.h"
 
 namespace wfb {
@@ -75,7 +75,8 @@ __global__ __launch_bounds__(kFinThreads) void argmax_finalize_kernel(const uint
   }
 }
 
-template <int XT, int WT, int MM>
+// NP: groups of 8 rows a wave takes at once (the dot-product path; the other takes one).
+template <int XT, int WT, int MM, int NP>
 __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x, int64_t ldx,
                                                       const void* __restrict__ gamma, int gdt, float eps,
                                                       const void* __restrict__ W, int64_t ldw, int m, int n, int h,
@@ -203,7 +204,6 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const void* __restrict__ x
   constexpr int U = 4;
   const int row0 = blockIdx.x * 64 + w * 16 + rsub;
   if constexpr (DOT) {
-    constexpr int NP = MM == 1 ? 1 : 2;  // row groups at once
 #pragma unroll
     for (int p0 = 0; p0 < 2; p0 += NP) {
       float acc[NP][MM];
@@ -306,15 +306,32 @@ template <int XT, int WT>
 hipError_t launch_head_t(const void* x, int64_t ldx, const void* gamma, int gdt, float eps, const void* w, int64_t ldw,
                          int m, int n, int h, float* logits, int64_t ldo, uint64_t* parts, hipStream_t s) {
   const dim3 grid((n + 63) / 64);
-  const size_t lds = (size_t)m * h * (XT == WFB_BF16 && WT == WFB_BF16 ? 2 : 4);
-#define WFB_HEAD(MMV) \
-  hipLaunchKernelGGL((lm_head_kernel<XT, WT, MMV>), grid, dim3(256), lds, s, x, ldx, gamma, gdt, eps, w, ldw, m, n, h, \
+  constexpr bool DOT = XT == WFB_BF16 && WT == WFB_BF16;
+  // (one token's rows ask for the LDS of fp32 values: with half of it more workgroups stream rows of 16 KB at once,
+  // 128256 x 8192 370 against 352 us)
+  const size_t lds = (size_t)m * h * (DOT && m > 1 ? 2 : 4);
+#define WFB_HEAD(MMV, NP) \
+  hipLaunchKernelGGL((lm_head_kernel<XT, WT, MMV, NP>), grid, dim3(256), lds, s, x, ldx, gamma, gdt, eps, w, ldw, m, n, h, \
                      logits, ldo, parts)
-  if (m <= 1) WFB_HEAD(1);
-  else if (m <= 2) WFB_HEAD(2);
-  else if (m <= 4) WFB_HEAD(4);
-  else if (m <= 8) WFB_HEAD(8);
-  else WFB_HEAD(16);
+  // Two row groups share each read of the tokens, but stream 16 rows a wave at once, which costs more where the rows lie
+  // a multiple of 8 KB apart and many workgroups stream, and where a third workgroup comes to some CUs only (cold
+  // weights on MI355X, two groups against one, us: 33333 x 4096 at M = 2 / 3 / 4 74.7 / 79.5 / 83.5 against 63.2 / 66.3 /
+  // 72.3, 65536 x 4096 at M = 4 119.6 against 111.5, 128256 x 4096 214 against 203; 33333 x 3584 at M = 2 60.9 against
+  // 55.7, x 2560 46.5 against 43.8; the other way 28672 x 4096 at M = 4 62.4 against 66.8, 49152 x 2560 at M = 2 54.1
+  // against 56.3, 128256 x 2560 at M = 4 133 against 143)
+  if constexpr (DOT) {
+    if (m > 1 && m <= 4 && n > 32768 && (h % 4096 == 0 || (h >= 2560 && n <= 40960))) {
+      if (m <= 2) WFB_HEAD(2, 1);
+      else WFB_HEAD(4, 1);
+      return hipGetLastError();
+    }
+  }
+  constexpr int NP = DOT ? 2 : 1;
+  if (m <= 1) WFB_HEAD(1, 1);
+  else if (m <= 2) WFB_HEAD(2, NP);
+  else if (m <= 4) WFB_HEAD(4, NP);
+  else if (m <= 8) WFB_HEAD(8, NP);
+  else WFB_HEAD(16, NP);
 #undef WFB_HEAD
   return hipGetLastError();
 }
