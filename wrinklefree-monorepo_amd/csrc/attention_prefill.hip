@@ -26,11 +26,12 @@
 // of softmax and conversion, 512 of them the 32 exponentials; counters at 4096 tokens, 32/8 heads of 128: MFMA busy
 // 55%, VALU 49% of the cycles of busy CUs.  32 queries per wave halve the LDS reads and the issue slots per product of
 // the 16-query form, which was LDS-bound; fragments are read 4 ahead of their products; the exponentials of a step run
-// under the products of the step before.  4096 tokens, 32/8 heads of 128: 388 -> 253 us; 8 x 2048 691 -> 498; 8 x 256
-// 36.4 -> 29.2; 2048 tokens of 40/8 heads 222 -> 113; 4096 of 9/3 heads of 64 160 -> 89 (one buffer, back to back on
-// one box; on buffers in turn the first is 341 -> 209 us, 655 TFLOP/s).
-// Measured without gain: K and V^T staged through registers as in the 16-token form (260 us; the transposing reads
-// make it no slower and free 32 registers), 32-key blocks at 3 waves per SIMD (25 spills, 307 us).
+// under the products of the step before.  Whole calls in a graph, buffers in turn, against the 16-token form: 4096
+// tokens, 32/8 heads of 128 357 -> 217 us (211 in a stream of calls: 650 TFLOP/s); 8 x 2048 637 -> 436; 8 x 256 29.4 ->
+// 23.3; 2048 tokens of 40/8 heads 204 -> 93; 4096 of 9/3 heads of 64 147 -> 79.
+// Measured without gain: K and V^T staged through registers as in the 16-token form (260 against 253 us of the kernel
+// as it was then; the transposing reads make it no slower and free 32 registers), 32-key blocks at 3 waves per SIMD (25
+// spills, 307 us).
 #include "wfb_common.h"
 
 namespace wfb {

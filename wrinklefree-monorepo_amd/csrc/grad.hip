@@ -7,14 +7,14 @@
 //   grad_w[n, k] = sum_m (g[m, n] * a_scale[m]) * q[m, k]          q an int8 code
 // Both run as C[i, j] = alpha * sum_p sum_c A_p[i, c] * B[j, c] with bf16 operands and fp32 accumulators.  t and
 // q are exact in bf16.  An fp32 factor enters as three bf16 planes cut off its bits (8 + 8 + 8 significant bits:
-// the planes sum to the value exactly, see split3), so every product is exact in fp32 and the only roundings are
-// those of the fp32 sums and of g * a_scale -- the ones an fp32 product has.  A bf16 gradient is its own single
-// plane in grad_x.
+// the planes sum to the value exactly, see split3 for where), so every product is exact in fp32 and the only roundings
+// are those of the fp32 sums and of g * a_scale (an fp32 product would round q * a_scale instead: where g * a_scale
+// leaves fp32's range, a code of 0 gives NaN).  A bf16 gradient is its own single plane in grad_x.
 //
 // Bound by the matrix cores: one pass over grad_x and three over grad_w instead of fp32 products, which run at a
-// sixteenth of the bf16 rate.  2048 tokens, 2560 -> 6912, bf16 (traced): grad_x 549 -> 88 us + 12 for its three
-// partial sums, grad_w 549 -> 189 + 6 us, the layout kernels 40 us in place of 160 us of conversions and transposes;
-// forward and backward 1396 -> 412 us.
+// sixteenth of the bf16 rate.  2048 tokens, 2560 -> 6912, bf16 (traced): grad_x 549 -> 87 us + 12 for its three
+// partial sums, grad_w 549 -> 180 + 7 us, the layout kernels 40 us in place of 160 us of conversions and transposes;
+// the whole step 1364 -> 397 us.
 //
 // Two steps.  Layout kernels write the operands with the summed index contiguous (the ternary codes and the int8
 // codes transposed to bf16; g * a_scale transposed and split), zero-padded to whole stages; then the tile kernel.
@@ -30,7 +30,7 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-// v = p[0] + p[1] + p[2] exactly (for |v| above 2^-110; below, the last bits of a plane may be subnormal): each
+// v = p[0] + p[1] + p[2] exactly for |v| above 2^-110 (below, bits under 2^-133, the smallest bf16, are cut off): each
 // plane is the top 16 bits of what is left, by truncation, so none overflows and each remainder is exact.  An
 // infinite v has the planes v, 0, 0 and a NaN NaN, 0, 0: they reach the product as they are.
 __device__ __forceinline__ void split3(float v, uint16_t (&p)[3]) {
@@ -490,7 +490,7 @@ struct Plan {
 // runs it in less than the time of a full one) and the partial sums written and read back.  Swept on MI355X over
 // every (variant, split of all tiles) of 18 shapes from 1 x 576 x 576 to 4096^3, both products: the estimate's pick
 // is within 8% of the fastest on all but four, within 15% there.  Splitting only the tiles past the last full round
-// (28 of 540 at 2048 x 6912 x 2560) took grad_w there from 200 us and 26 for all tiles' sums to 189 and 6.
+// (28 of 540 at 2048 x 6912 x 2560) took grad_w there from 200 us and 26 for all tiles' sums to 180-189 and 7.
 Plan plan(int planes, int64_t I, int64_t J, int64_t C) {
   Plan best{-1, 0, 0, 1};
   double best_us = 0;

@@ -6,8 +6,9 @@
 // blockIdx.x, + gridDim.x, ...; a thread keeps its columns' part of grad_w in registers over all of them, and the
 // row's elements between the two sums and the output, so every element is read once.  Bound by the two block
 // reductions of a row at small M and by memory at large M: the next row's loads are requested before this row's
-// reductions.  Against the torch composition: 501 x 1536 fp32 185 -> 17 us, 2048 x 2560 bf16 194 -> 19 us, 8192 x 6912
-// bf16 1335 -> 138 us (3.3 TB/s).
+// reductions.  Against the torch composition, with the column sums: 501 x 1536 fp32 185 -> 11 us, 2048 x 2560 bf16 194
+// -> 19 us, 8192 x 6912 bf16 1335 -> 139 us (3.3 TB/s).  Rows above 8192 hold 422 registers a thread, one workgroup per
+// CU: 8192 x 14336 bf16 384 us (2.5 TB/s), fp32 289 (4.9), 501 x 14336 bf16 41.
 #include "wfb_common.h"
 
 namespace wfb {
@@ -140,7 +141,7 @@ hipError_t launch_t(const void* x, const void* w, int wdt, const float* g, float
 }
 
 // out[c] = sum over the rows of part[rows][cols], in a fixed order: 16 rows of threads each take every 16th row,
-// 16 loads in flight, then a tree.  16 x 16 threads: 16 columns per workgroup.
+// 8 loads in flight, then a tree.  16 x 16 threads: 16 columns per workgroup.
 __global__ __launch_bounds__(256) void column_sum_kernel(const float* __restrict__ part, int rows, int64_t cols,
                                                          void* __restrict__ out, int out_dtype) {
   __shared__ float red[16][17];
@@ -179,7 +180,8 @@ hipError_t launch_column_sum(const float* part, int rows, int64_t cols, void* ou
   return hipGetLastError();
 }
 
-// Two workgroups per CU walk the rows; each leaves one row of partial sums.
+// 512 workgroups walk the rows, two per CU (one after the other where a row is longer than 8192); each leaves one row of
+// partial sums.
 int norm_grad_parts(int64_t m) { return (int)(m < 512 ? m : 512); }
 
 hipError_t launch_norm_grad(const void* x, int dt, const void* w, int wdt, const float* g, float eps, int64_t m,
