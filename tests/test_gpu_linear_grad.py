@@ -91,6 +91,19 @@ def test_every_tile_form_matches_float64(pkg, dev, which, dtype, size, form):
     assert _rel(got, want) <= tol
 
 
+@pytest.mark.parametrize("m,k", [(1, 20), (6, 20), (70, 131), (65, 127)])
+def test_grad_w_codes_may_end_with_their_last_row(pkg, dev, m, k):
+    """Rows 16-byte aligned whose storage ends with the last row's codes (no padding behind them)."""
+    ops, n, ld = pkg.ops, 40, (k + 15) // 16 * 16
+    g = torch.Generator(device=dev).manual_seed(k)
+    flat = torch.randint(-127, 128, ((m - 1) * ld + k,), generator=g, device=dev, dtype=torch.int8)
+    codes = flat.as_strided((m, k), (ld, 1))
+    a_scale = torch.rand(m, generator=g, device=dev) + 0.1
+    gy = torch.randn((m, n), generator=g, device=dev)
+    want = (gy.double() * a_scale.double()[:, None]).t().contiguous() @ codes.double()
+    assert _rel(ops.linear_grad_w(codes, a_scale, gy, k, torch.float32), want) <= 1e-6
+
+
 @pytest.mark.parametrize("m", [520, 1030])
 def test_grad_w_splits_only_the_last_tiles(pkg, dev, m):
     """605 tiles: 512 summed by one workgroup each and the last 93 in 2 or 5 parts, at ragged edges of both."""

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void grad_planes_kernel(const void* __restrict
 }
 
 // int8 codes q[m][k] as bf16 dst[k][m], rows of mp elements (m >= M: zeros).  VEC: 16 codes per load (rows 16-byte
-// aligned and ldq >= K rounded up to 16).
+// aligned); a row's last codes, fewer than 16, one at a time: nothing has to lie behind the last row's.
 template <bool VEC>
 __global__ __launch_bounds__(256) void codes_t_kernel(const int8_t* __restrict__ q, int64_t ldq, int64_t M, int64_t K,
                                                       int64_t mp, uint16_t* __restrict__ dst) {
@@ -129,12 +129,12 @@ __global__ __launch_bounds__(256) void codes_t_kernel(const int8_t* __restrict__
   const int r = threadIdx.x >> 2, c = 16 * (threadIdx.x & 3);  // 16 codes of row r
   const int64_t m = m0 + r, row = (m < M ? m : M - 1) * ldq;
   uint32_t v[4] = {0, 0, 0, 0};
-  if (VEC) {
-    if (m < M && k0 + c < K) {
+  if (VEC && k0 + c + 16 <= K) {
+    if (m < M) {
       const uint4 x = *reinterpret_cast<const uint4*>(q + row + k0 + c);
       v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
     }
-  } else {
+  } else if (k0 + c < K) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int64_t k = k0 + c + e;
