@@ -299,6 +299,27 @@ def test_rmsnorm_grad_matches_float64(pkg, dev, m, h, dtype):
     assert only[0] is None and torch.equal(only[1], got[1])
 
 
+def test_gradient_ops_refuse_what_they_cannot_read(pkg, dev):
+    ops = pkg.ops
+    qw, scale = torch.zeros((8, 64), dtype=torch.uint8, device=dev), torch.ones(1, device=dev)
+    gy, codes = torch.zeros((4, 8), device=dev), torch.zeros((4, 256), dtype=torch.int8, device=dev)
+    a_scale, f32 = torch.ones(4, device=dev), torch.float32
+    for bad in ((qw.int(), scale, gy, 256, f32), (qw, scale.double(), gy, 256, f32), (qw, scale, gy[:, :7], 256, f32),
+                (qw, scale, gy, 257, f32), (qw, scale, gy, 0, f32), (qw, scale, gy.double(), 256, f32),
+                (qw, scale, gy, 256, torch.float64), (qw.cpu(), scale, gy, 256, f32)):
+        with pytest.raises(RuntimeError):
+            ops.linear_grad_x(*bad)
+    for bad in ((codes.short(), a_scale, gy, 256, f32), (codes.t().contiguous().t(), a_scale, gy, 256, f32),
+                (codes[:3], a_scale, gy, 256, f32), (codes, a_scale[:3], gy, 256, f32), (codes, a_scale, gy, 257, f32),
+                (codes, a_scale, gy, 256, f32, torch.int32), (codes.cpu(), a_scale, gy, 256, f32)):
+        with pytest.raises(RuntimeError):
+            ops.linear_grad_w(*bad)
+    x, w = torch.zeros((4, 256), device=dev), torch.ones(256, device=dev)
+    for bad in ((x, w, x.bfloat16()), (x, w[:128], x), (x, w, x[:3]), (x.double(), w, x), (x[:, :252].contiguous(), w[:252], x[:, :252].contiguous())):
+        with pytest.raises(RuntimeError):
+            ops.rmsnorm_grad(*bad, 1e-6)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("h", [8, 1000, 16384])
 def test_rmsnorm_grad_of_no_rows_is_zero(pkg, dev, dtype, h):

@@ -701,6 +701,8 @@ def linear_grad_x(packed_weights: torch.Tensor, scale: torch.Tensor, grad: torch
     n, kb = packed_weights.shape
     grad = grad.contiguous()
     dev = _require_gpu(name, packed_weights, scale, grad)
+    if packed_weights.dtype != torch.uint8:
+        raise RuntimeError(f"{name}: packed_weights must be uint8")
     if grad.dim() != 2 or grad.shape[1] != n or not 0 < in_features <= kb * 4:
         raise RuntimeError(f"{name}: grad must be [tokens, {n}] and in_features at most {kb * 4}")
     if scale.dtype != torch.float32 or scale.numel() != 1 or out_dtype not in _DT:
