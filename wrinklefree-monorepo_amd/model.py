@@ -101,7 +101,7 @@ class HipBackend:
     ``fused=True``: the projections of a group (q|k|v, gate|up) run as one segmented launch on their
     concatenated weights, residual adds ride in the o/down epilogues, and for decode batches the
     norm + quantiser before q|k|v and o runs in the linear's prologue where that is measured faster
-    (``rmsnorm_linear_preferred``, a rule by rows): a Llama-3-8B decode layer takes 8 kernel launches (norm+q|k|v,
+    (``rmsnorm_linear_preferred``): a Llama-3-8B decode layer takes 8 kernel launches (norm+q|k|v,
     attention and its split combine, SubLN+o+residual, norm+quant, gate|up, act+SubLN+quant,
     down+residual) instead of 12."""
 

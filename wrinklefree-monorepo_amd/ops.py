@@ -39,8 +39,8 @@ def check_kernel_available() -> bool:
 
 
 # What every call pays on the host.  A small call is bound by it, not by its kernels: one token through a 576 x 576
-# BitLinear is two launches, 30.2 us a call with a device guard, a stream object and pointer boxes around each and
-# 22.2 without (the fused MLP of one token 45.2 -> 32.7).  Pointers and streams go to the C entry points as plain
+# BitLinear is two launches, 30.6 us a call with a device guard, a stream object and pointer boxes around each and
+# 23.1 without (the fused MLP of one token 47.2 -> 34.2).  Pointers and streams go to the C entry points as plain
 # integers (their argument types are declared), the stream comes from torch's raw accessor, and the device guard is
 # entered only for a device that is not the current one.
 
